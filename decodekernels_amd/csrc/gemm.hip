@@ -44,6 +44,8 @@ constexpr int kRsrcWord3 = 0x00020000;
 // Byte offset that is outside every buffer resource used here: loads there
 // return zero without touching memory.
 constexpr int kOutOfRange = 0x7fffffff;
+// The same for offsets to which a K offset may be added, vector or scalar (both below 2^31; unsigned).
+constexpr unsigned kNowhere = 0x80000000u;
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* base, int64_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0,
@@ -367,31 +369,152 @@ __device__ __forceinline__ void dma_tile_of(int id, int tiles_m, int tiles_n, in
   tn = (pid % per_group) / gm;
 }
 
+// The order in which a workgroup takes the K slices of [kb, kb + 64 ktiles):
+// from slice `rot` on, round to slice rot - 1 (rot = 0: in order).
+struct KWalk {
+  int kb, end, ktiles, rot;
+  __device__ __forceinline__ KWalk(int kb_, int ktiles_, int rot_)
+      : kb(kb_), end(kb_ + ktiles_ * kDmaBK), ktiles(ktiles_), rot(ktiles_ > 0 ? rot_ % ktiles_ : 0) {}
+  // First column of the walk's slice t; past the range for t >= ktiles.
+  __device__ __forceinline__ int at(int t) const {
+    const int r = t + rot;
+    return kb + (t < ktiles && r >= ktiles ? r - ktiles : r) * kDmaBK;
+  }
+  // First column of the slice after the one at column k0 (before the walk's end).
+  __device__ __forceinline__ int after(int k0) const { return k0 + kDmaBK == end ? kb : k0 + kDmaBK; }
+};
+
+// Bytes of a wave's output tile staged in LDS: 16 TM rows of 16 TN 16-bit
+// columns, padded by 16 bytes a row.
+template <int TM, int TN>
+constexpr int stage_bytes() {
+  return 16 * TM * (32 * TN + 16);
+}
+
+// Writes a wave's 16 TM x 16 TN output tile at (m0, n0): acc[i][j] lane l, reg
+// r = C[m0 + 16 i + l % 16][n0 + 16 j + 4 (l / 16) + r]. With part != nullptr
+// the fp32 sums go to part[blockIdx.y][M][N] without the bias; else bias and
+// rounding, through LDS. Called by every wave of the workgroup, with no loads
+// into LDS in flight; `lds` holds stage_bytes() for each wave.
+template <typename E, int TM, int TN>
+__device__ __forceinline__ void store_tile(const f32x4 (&acc)[TM][TN], u32x4* lds, int lane, int wave, int m0, int n0,
+                                           const uint16_t* __restrict__ bias, uint16_t* __restrict__ C, int M, int N,
+                                           int ldc, int vec_store, float* __restrict__ part) {
+  constexpr int kPitch = 32 * TN + 16;  // bytes per staged output row
+  const int l16 = lane % 16;
+  const int lg = lane / 16;
+  if (part != nullptr) {  // fp32 partial tile, no bias
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int n = n0 + 16 * j + 4 * lg;
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const int m = m0 + 16 * i + l16;
+        if (m >= M) continue;
+        float* prow = part + (static_cast<int64_t>(blockIdx.y) * M + m) * N;
+        if (N % 4 == 0 && n + 3 < N) {
+          *reinterpret_cast<f32x4*>(prow + n) = acc[i][j];
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (n + r < N) prow[n + r] = acc[i][j][r];
+        }
+      }
+    }
+    return;
+  }
+
+  // Every bias value this lane adds, loaded before any store, with clamped
+  // addresses and no branch per element so that the loads issue together.
+  // (Loaded one at a time under a bounds branch, each was waited for behind
+  // the stores before it: up to 6 us at M = N = 4096.) Columns past N are
+  // never stored, so their clamped values do not matter.
+  float bj[TN][4];
+  if (bias != nullptr) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int n = n0 + 16 * j + 4 * lg;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) bj[j][r] = E::to_float(bias[min(n + r, N - 1)]);
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) bj[j][r] = 0.0f;
+  }
+
+  // The output goes through LDS: each wave writes its tile into its own part
+  // of the allocation in the MFMA layout (8 bytes per lane), then
+  // reads it back row by row, 16 bytes per lane, so a store writes whole row
+  // segments instead of 32-byte pieces of 16 rows. Rows are padded by 16 bytes.
+  constexpr int kNc = 2 * TN;  // 16-byte chunks per tile row
+  char* stg = reinterpret_cast<char*>(lds) + wave * stage_bytes<TM, TN>();
+  __syncthreads();  // every wave is done with the ring
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const int row = 16 * i + l16;
+      const int c = 2 * j + lg / 2;
+      float v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = acc[i][j][r] + bj[j][r];
+      *reinterpret_cast<u32x2*>(stg + row * kPitch + c * 16 + (lg % 2) * 8) =
+          u32x2{pack2<E>(v[0], v[1]), pack2<E>(v[2], v[3])};
+    }
+  }
+  __syncthreads();  // the tile's rows come from the other lanes of the wave
+  constexpr int kChunks = 16 * TM * kNc;  // 16-byte chunks of a wave's tile
+#pragma unroll
+  for (int it = 0; it < (kChunks + kWave - 1) / kWave; ++it) {
+    const int idx = it * kWave + lane;
+    if (kChunks % kWave != 0 && idx >= kChunks) break;  // last pass part-filled (192 x 224: 10.5 passes)
+    const int row = idx / kNc;
+    const int c = idx % kNc;
+    const u32x4 val = *reinterpret_cast<const u32x4*>(stg + row * kPitch + c * 16);
+    const int m = m0 + row;
+    const int n = n0 + 8 * c;
+    if (m >= M) continue;
+    uint16_t* crow = C + static_cast<int64_t>(m) * ldc;
+    if (vec_store == 2 && n + 7 < N) {
+      *reinterpret_cast<u32x4*>(crow + n) = val;
+    } else if (vec_store == 1 && n + 7 < N) {
+      *reinterpret_cast<u32x2*>(crow + n) = u32x2{val[0], val[1]};
+      *reinterpret_cast<u32x2*>(crow + n + 4) = u32x2{val[2], val[3]};
+    } else {
+#pragma unroll
+      for (int r = 0; r < 8; ++r)
+        if (n + r < N) crow[n + r] = static_cast<uint16_t>(val[r / 2] >> (16 * (r % 2)));
+    }
+  }
+}
+
+// The ring body: every wave waits for slice t, meets the others at a barrier,
+// starts slice t + STAGES - 1 and multiplies.
 template <typename E, int BM, int BN, int WM, int WN, int STAGES>
-__global__ __launch_bounds__(WM * WN * kWave) void gemm_dma_kernel(const uint16_t* __restrict__ A,
-                                                                   const uint16_t* __restrict__ B,
-                                                                   const uint16_t* __restrict__ bias,
-                                                                   uint16_t* __restrict__ C, int M, int N, int K,
-                                                                   int lda, int ldb, int ldc, int vec_store,
-                                                                   float* __restrict__ part, int k_split) {
+__device__ __forceinline__ void ring_tile(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
+                                          const uint16_t* __restrict__ bias, uint16_t* __restrict__ C, int M, int N,
+                                          int K, int lda, int ldb, int ldc, int vec_store, float* __restrict__ part,
+                                          int k_split, int rot_step) {
   constexpr int NW = WM * WN;
   constexpr int TM = BM / WM / 16;  // 16-row fragments per wave
   constexpr int TN = BN / WN / 16;
   constexpr int LA = BM / 8 / NW;   // 1 KB DMA loads per wave per slice
   // B's 8-row load groups need not divide among the waves (256 x 224: 28 groups
-  // for 8 waves); the waves past the last group skip their final load.
+  // for 8 waves). A wave past the last group skips its final load where the
+  // ring's waits are vmcnt(0) (2 stages); else it issues one that moves nothing,
+  // aimed at a spare 1 KB, so that every wave has the same count in flight.
   constexpr int kGroupsB = BN / 8;
   constexpr int LB = (kGroupsB + NW - 1) / NW;
   constexpr bool kTailB = kGroupsB % NW != 0;
   constexpr int kSlice = (BM + BN) * 8;  // u32x4 per slice
   static_assert(BM % (8 * NW) == 0 && BN % 8 == 0 && TM >= 1 && TN >= 1 && BN % (16 * WN) == 0, "tile shape");
   static_assert(STAGES >= 2 && (STAGES - 2) * (LA + LB) < 64, "vmcnt range");
-  // With uneven B loads the waves have different counts in flight, which only
-  // a 2-stage ring's vmcnt(0) waits allow.
-  static_assert(!kTailB || STAGES == 2, "uneven B loads need STAGES == 2");
-  constexpr int kStagePitch = BN / WN * 2 + 16;         // bytes per staged output row
-  constexpr int kStageWave = BM / WM * kStagePitch;     // bytes of one wave's staged tile
-  constexpr int kLdsU4 = STAGES * kSlice > NW * kStageWave / 16 ? STAGES * kSlice : NW * kStageWave / 16;
+  constexpr int kStageWave = stage_bytes<TM, TN>();
+  constexpr bool kSpare = kTailB && STAGES > 2;
+  constexpr int kRingU4 = STAGES * kSlice + (kSpare ? 64 : 0);
+  constexpr int kLdsU4 = kRingU4 > NW * kStageWave / 16 ? kRingU4 : NW * kStageWave / 16;
   static_assert(kLdsU4 * 16 <= 160 * 1024, "LDS of one workgroup (gfx950: 160 KB)");
   __shared__ u32x4 lds[kLdsU4];
 
@@ -422,41 +545,47 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_dma_kernel(const uint16_
       rsrc(B + static_cast<int64_t>(n0) * ldb, (static_cast<int64_t>(rows_b - 1) * ldb + K) * 2);
 
   // DMA lane roles: load j of this wave fills tile rows 8 g .. 8 g + 7 (g = wave + j NW);
-  // lane l writes position l % 8 of row 8 g + l / 8, i.e. chunk (l % 8) ^ swz(row).
-  int offa[LA], ka[LA], offb[LB], kbc[LB];
+  // lane l writes position l % 8 of row 8 g + l / 8, i.e. chunk (l % 8) ^ swz(row) = (l % 8) ^ (l / 8).
+  const int kc = 8 * ((lane % 8) ^ (lane / 8));  // first column of this lane's 16 bytes in a slice
+  unsigned offa[LA], offb[LB];
 #pragma unroll
   for (int j = 0; j < LA; ++j) {
     const int r = 8 * (wave + j * NW) + lane / 8;
-    const int c = (lane % 8) ^ swz(r);
-    ka[j] = 8 * c;
-    offa[j] = r < rows_a ? r * lda * 2 + 16 * c : kOutOfRange;
+    offa[j] = r < rows_a ? static_cast<unsigned>(r * lda * 2 + 2 * kc) : kNowhere;
   }
 #pragma unroll
   for (int j = 0; j < LB; ++j) {
     const int r = 8 * (wave + j * NW) + lane / 8;
-    const int c = (lane % 8) ^ swz(r);
-    kbc[j] = 8 * c;
-    offb[j] = r < rows_b && r < BN ? r * ldb * 2 + 16 * c : kOutOfRange;
+    offb[j] = r < rows_b && r < BN ? static_cast<unsigned>(r * ldb * 2 + 2 * kc) : kNowhere;
   }
-  // Issued for every slice index, also past the last one (those lanes are out
-  // of range and move no data), so each wave keeps the same count in flight
-  // from slice to slice.
-  auto issue = [&](int t, int buf) {
-    const int k0 = kb + t * kDmaBK;
+  const int ktiles = (ke - kb + kDmaBK - 1) / kDmaBK;
+  const int full = (ke - kb) / kDmaBK;  // slices that lie wholly inside the K range
+  const KWalk walk(kb, ktiles, full == ktiles ? tn * rot_step : 0);
+  // Slice t of the walk into ring buffer `buf`. Checked: also for slices that
+  // end past the K range, or start there (those lanes are out of range and move
+  // no data), so that each wave keeps the same count in flight from slice to
+  // slice. Whole slices take their K offset as the load's scalar offset, which
+  // leaves no vector arithmetic in the steady loop, and `k0` steps with the
+  // walk (a compare and a select per slice).
+  auto issue = [&](bool checked, int k0, int buf) {
     u32x4* base = lds + buf * kSlice;
+    const bool in = k0 + kc < ke;
 #pragma unroll
     for (int j = 0; j < LA; ++j) {
-      const int off = (offa[j] != kOutOfRange && k0 + ka[j] < ke) ? offa[j] + 2 * k0 : kOutOfRange;
+      const int off = static_cast<int>(checked ? (in ? offa[j] + 2 * k0 : kNowhere) : offa[j]);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          ra, (__attribute__((address_space(3))) void*)(base + (wave + j * NW) * 64), 16, off, 0, 0, 0);
+          ra, (__attribute__((address_space(3))) void*)(base + (wave + j * NW) * 64), 16, off, checked ? 0 : 2 * k0, 0, 0);
     }
 #pragma unroll
     for (int j = 0; j < LB; ++j) {
-      // A wave past B's last load group issues nothing (its LDS target would be past the slice).
-      if (kTailB && j == LB - 1 && wave + j * NW >= kGroupsB) break;
-      const int off = (offb[j] != kOutOfRange && k0 + kbc[j] < ke) ? offb[j] + 2 * k0 : kOutOfRange;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rb, (__attribute__((address_space(3))) void*)(base + BM * 8 + (wave + j * NW) * 64), 16, off, 0, 0, 0);
+      u32x4* to = base + BM * 8 + (wave + j * NW) * 64;
+      if (kTailB && j == LB - 1 && wave + j * NW >= kGroupsB) {  // past B's last load group (offb is out of range)
+        if (!kSpare) break;
+        to = lds + STAGES * kSlice;
+      }
+      const int off = static_cast<int>(checked ? (in ? offb[j] + 2 * k0 : kNowhere) : offb[j]);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (__attribute__((address_space(3))) void*)to, 16, off,
+                                               checked ? 0 : 2 * k0, 0, 0);
     }
   };
 
@@ -481,152 +610,359 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_dma_kernel(const uint16_
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  const int ktiles = (ke - kb + kDmaBK - 1) / kDmaBK;
 #pragma unroll
-  for (int s = 0; s < STAGES - 1; ++s) issue(s, s);
+  for (int s = 0; s < STAGES - 1; ++s) issue(true, walk.at(s), s);
 
   // vmcnt(n) with expcnt / lgkmcnt left at their maxima (gfx9 encoding).
   constexpr int kWaitN = (STAGES - 2) * (LA + LB);
   constexpr int kWaitImm = (kWaitN & 15) | ((kWaitN >> 4) << 14) | (7 << 4) | (15 << 8);
 
-  for (int t0 = 0; t0 < ktiles; t0 += STAGES) {
+  // The next slice, in ring buffer u; the loads of the slice STAGES - 1 later start at column k0.
+  auto step = [&](bool checked, int k0, int u) {
+    // This wave's loads of the slice have landed; the barrier extends that to
+    // every wave and ensures all reads of the buffer refilled next are done.
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(kWaitImm);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    issue(checked, k0, (u + STAGES - 1) % STAGES);
+    const u32x4* sl = lds + u * kSlice;
+    // Small tiles read both halves' fragments before the first MFMA, one LDS
+    // round trip a slice instead of two: o_proj at M = 250 (64 x 64) 16.4 -> 15.6
+    // us, qkv at M = 512 (128 x 128) 32.9 -> 30.8. Larger ones have no registers
+    // for it.
+    constexpr int kHalves = TM + TN <= 7 ? 2 : 1;
+    u32x4 af[kHalves][TM], bf[kHalves][TN];
+    auto read = [&](int h) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i) af[h % kHalves][i] = sl[ia[i][h]];
+#pragma unroll
+      for (int j = 0; j < TN; ++j) bf[h % kHalves][j] = sl[ib[j][h]];
+    };
+    if (kHalves == 2) {
+      read(0);
+      read(1);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if (kHalves == 1) read(h);
+      // A wave that has its fragments issues its MFMAs ahead of the other
+      // wave on the SIMD, which meanwhile reads its own: the two drift
+      // out of phase instead of reading and multiplying in lockstep
+      // (measured 1-4% at M = 1024 / 4096).
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          acc[i][j] = E::mfma_16x16x32(bf[h % kHalves][j], af[h % kHalves][i], acc[i][j]);
+      __builtin_amdgcn_s_setprio(0);
+    }
+  };
+  int t0 = 0;
+  int k0 = walk.at(STAGES - 1);
+  for (; t0 + 2 * STAGES - 2 < full; t0 += STAGES) {
 #pragma unroll
     for (int u = 0; u < STAGES; ++u) {
-      if (t0 + u < ktiles) {
-        // This wave's loads of slice t0 + u have landed; the barrier extends that
-        // to every wave and ensures all reads of the buffer refilled next are done.
-        __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_waitcnt(kWaitImm);
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_sched_barrier(0);
-        issue(t0 + u + STAGES - 1, (u + STAGES - 1) % STAGES);
-        const u32x4* sl = lds + u * kSlice;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          u32x4 af[TM], bf[TN];
-#pragma unroll
-          for (int i = 0; i < TM; ++i) af[i] = sl[ia[i][h]];
-#pragma unroll
-          for (int j = 0; j < TN; ++j) bf[j] = sl[ib[j][h]];
-          // A wave that has its fragments issues its MFMAs ahead of the other
-          // wave on the SIMD, which meanwhile reads its own: the two drift
-          // out of phase instead of reading and multiplying in lockstep
-          // (measured 1-4% at M = 1024 / 4096).
-          __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-          for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j) acc[i][j] = E::mfma_16x16x32(bf[j], af[i], acc[i][j]);
-          __builtin_amdgcn_s_setprio(0);
-        }
-      }
+      step(false, k0, u);
+      k0 = walk.after(k0);
     }
+  }
+  for (; t0 < ktiles; t0 += STAGES) {
+#pragma unroll
+    for (int u = 0; u < STAGES; ++u)
+      if (t0 + u < ktiles) step(true, walk.at(t0 + u + STAGES - 1), u);
   }
 
   // The loads issued past the last slice move no data, but none may still be
   // in flight into this workgroup's LDS when it exits.
   __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));
 
-  // acc[i][j] lane l, reg r = C[m0 + wm BM/WM + 16 i + l % 16][n0 + wn BN/WN + 16 j + 4 (l / 16) + r].
-  if (part != nullptr) {  // fp32 partial tile, no bias
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int n = n0 + wn * (BN / WN) + 16 * j + 4 * lg;
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        const int m = m0 + wm * (BM / WM) + 16 * i + l16;
-        if (m >= M) continue;
-        float* prow = part + (static_cast<int64_t>(blockIdx.y) * M + m) * N;
-        if (N % 4 == 0 && n + 3 < N) {
-          *reinterpret_cast<f32x4*>(prow + n) = acc[i][j];
-        } else {
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (n + r < N) prow[n + r] = acc[i][j][r];
-        }
-      }
-    }
-    return;
-  }
-
-  // Every bias value this lane adds, loaded before any store, with clamped
-  // addresses and no branch per element so that the loads issue together.
-  // (Loaded one at a time under a bounds branch, each was waited for behind
-  // the stores before it: up to 6 us at M = N = 4096.) Columns past N are
-  // never stored, so their clamped values do not matter.
-  float bj[TN][4];
-  if (bias != nullptr) {
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int n = n0 + wn * (BN / WN) + 16 * j + 4 * lg;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) bj[j][r] = E::to_float(bias[min(n + r, N - 1)]);
-    }
-  } else {
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) bj[j][r] = 0.0f;
-  }
-
-  // The output goes through LDS: each wave writes its (BM/WM) x (BN/WN) tile
-  // into its own part of the ring in the MFMA layout (8 bytes per lane), then
-  // reads it back row by row, 16 bytes per lane, so a store writes whole row
-  // segments instead of 32-byte pieces of 16 rows. Rows are padded by 16 bytes.
-  constexpr int kNc = BN / WN / 8;  // 16-byte chunks per tile row
-  char* stg = reinterpret_cast<char*>(lds) + wave * kStageWave;
-  __syncthreads();  // every wave is done with the ring
-#pragma unroll
-  for (int j = 0; j < TN; ++j) {
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int row = 16 * i + l16;
-      const int c = 2 * j + lg / 2;
-      float v[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) v[r] = acc[i][j][r] + bj[j][r];
-      *reinterpret_cast<u32x2*>(stg + row * kStagePitch + c * 16 + (lg % 2) * 8) =
-          u32x2{pack2<E>(v[0], v[1]), pack2<E>(v[2], v[3])};
-    }
-  }
-  __syncthreads();  // the tile's rows come from the other lanes of the wave
-  constexpr int kChunks = (BM / WM) * kNc;  // 16-byte chunks of a wave's tile
-#pragma unroll
-  for (int it = 0; it < (kChunks + kWave - 1) / kWave; ++it) {
-    const int idx = it * kWave + lane;
-    if (kChunks % kWave != 0 && idx >= kChunks) break;  // last pass part-filled (192 x 224: 10.5 passes)
-    const int row = idx / kNc;
-    const int c = idx % kNc;
-    const u32x4 val = *reinterpret_cast<const u32x4*>(stg + row * kStagePitch + c * 16);
-    const int m = m0 + wm * (BM / WM) + row;
-    const int n = n0 + wn * (BN / WN) + 8 * c;
-    if (m >= M) continue;
-    uint16_t* crow = C + static_cast<int64_t>(m) * ldc;
-    if (vec_store == 2 && n + 7 < N) {
-      *reinterpret_cast<u32x4*>(crow + n) = val;
-    } else if (vec_store == 1 && n + 7 < N) {
-      *reinterpret_cast<u32x2*>(crow + n) = u32x2{val[0], val[1]};
-      *reinterpret_cast<u32x2*>(crow + n + 4) = u32x2{val[2], val[3]};
-    } else {
-#pragma unroll
-      for (int r = 0; r < 8; ++r)
-        if (n + r < N) crow[n + r] = static_cast<uint16_t>(val[r / 2] >> (16 * (r % 2)));
-    }
-  }
+  store_tile<E, TM, TN>(acc, lds, lane, wave, m0 + wm * (BM / WM), n0 + wn * (BN / WN), bias, C, M, N, ldc, vec_store, part);
 }
+
+// ---------------------------------------------------------------------------
+// Ping-pong body (256-row and 256-column tiles)
+// ---------------------------------------------------------------------------
+// The ring body reads a slice's fragments and multiplies them in turn, every
+// wave at once: per 256 x 256 slice the LDS reads and the MFMAs each take
+// about 2000 cycles, and 4000 passed. Here the two waves of a SIMD alternate:
+// while one multiplies (16 MFMAs, raised priority) the other reads its next
+// fragments and starts its share of the loads, with a barrier at every swap.
+// Waves 4-7 run one barrier behind waves 0-3.
+//
+// A slice's A and B are kept as two halves each: half i holds, for every wave
+// row (column) of the grid, its i-th 1/2 of the rows (columns), so a wave's
+// tile is four quadrants A_i x B_j and a slice four phases:
+//   read A0, x B0 | read B1, A0 x B1 | read A1, A1 x B1 | read the next B0, A1 x B0.
+// A half is refilled for slice t + 2 in the phase after the one that read it
+// last (B0, A0, B1, A1 in turn, one half per phase), so each load has seven
+// phases to land and the wait before each barrier leaves the newest six halves
+// in flight. Both hazards are closed by the barriers: a wave waits for its own
+// reads (lgkmcnt(0)) and for its own loads of the half read next (vmcnt)
+// before the first barrier of a phase, and the wave one barrier behind has
+// passed that wait before the other enters its next phase.
+//
+// What bounds it is the phase's memory part, so it holds nothing but the
+// reads, the loads and their LDS addresses: a whole slice's K offset is the
+// loads' scalar offset (with it in the vector offset, and compared with the K
+// range per lane, the 256 x 256 tile took 674 us on gate_up at M = 4096, with
+// the ring body 741; now 643, hipBLASLt 641, same run). M = N = 4096: K = 4096
+// 112.5 -> 93.2 us, K = 14336 383 -> 346 us. Loads alone take 256 us of the
+// latter, MFMAs alone 227 us. Waiting for the reads only when they are used,
+// without the raised priority, with the loads in two phases instead of four,
+// or starting each XCD at another K offset were all within 1%.
+//
+// A square tile's waves form a 2 x 4 grid (1-2% faster than 4 x 2).
+// A barrier that neither LDS reads nor loads into LDS are moved across.
+__device__ __forceinline__ void pp_barrier() {
+  __builtin_amdgcn_sched_barrier(0);
+  __asm__ volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  __asm__ volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// Waits for this wave's fragment reads and until at most VM of its loads into
+// LDS are in flight, then for the other waves.
+template <int VM>
+__device__ __forceinline__ void pp_wait_barrier() {
+  static_assert(VM < 64, "vmcnt range");
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt((VM & 15) | ((VM >> 4) << 14) | (7 << 4));
+  pp_barrier();
+}
+
+template <typename E, int BM, int BN, int GM, int GN>
+__device__ __forceinline__ void ping_pong_tile(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
+                                               const uint16_t* __restrict__ bias, uint16_t* __restrict__ C, int M,
+                                               int N, int K, int lda, int ldb, int ldc, int vec_store,
+                                               float* __restrict__ part, int k_split, int rot_step) {
+  constexpr int WM = BM == BN ? GN : GM;
+  constexpr int WN = BM == BN ? GM : GN;
+  constexpr int NW = WM * WN;
+  static_assert(NW == 8, "two waves per SIMD, one of each half of the workgroup");
+  constexpr int QR = BM / 2 / WM;  // rows of A (of B) of one half that a wave multiplies
+  constexpr int QC = BN / 2 / WN;
+  constexpr int QM = QR / 16;      // 16-row fragments of a half per wave
+  constexpr int QN = QC / 16;
+  static_assert(QR % 16 == 0 && QC % 16 == 0 && QM >= 1 && QN >= 1, "tile shape");
+  constexpr int kGroupsA = BM / 16;  // 8-row load groups of a half
+  constexpr int kGroupsB = BN / 16;
+  constexpr int LA = (kGroupsA + NW - 1) / NW;
+  constexpr int LB = (kGroupsB + NW - 1) / NW;
+  constexpr bool kTail = kGroupsA % NW != 0 || kGroupsB % NW != 0;
+  constexpr int kHalfA = BM / 2 * 8;  // u32x4 of a half
+  constexpr int kHalfB = BN / 2 * 8;
+  constexpr int kSlice = 2 * (kHalfA + kHalfB);
+  constexpr int kStage = NW * stage_bytes<2 * QM, 2 * QN>() / 16;
+  constexpr int kRing = 2 * kSlice + (kTail ? 64 : 0);
+  constexpr int kLdsU4 = kRing > kStage ? kRing : kStage;
+  static_assert(kLdsU4 * 16 <= 160 * 1024, "LDS of one workgroup (gfx950: 160 KB)");
+  __shared__ u32x4 lds[kLdsU4];
+
+  const int lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int wm = wave / WN;
+  const int wn = wave % WN;
+  const int l16 = lane % 16;
+  const int lg = lane / 16;
+
+  const int kb = part != nullptr ? static_cast<int>(blockIdx.y) * k_split : 0;
+  const int ke = part != nullptr ? min(K, kb + k_split) : K;
+  const int tiles_m = (M + BM - 1) / BM;
+  const int tiles_n = (N + BN - 1) / BN;
+  int tm, tn;
+  dma_tile_of<BM, BN>(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  const int m0 = tm * BM;
+  const int n0 = tn * BN;
+  const int rows_a = min(BM, M - m0);
+  const int rows_b = min(BN, N - n0);
+  const __amdgpu_buffer_rsrc_t ra =
+      rsrc(A + static_cast<int64_t>(m0) * lda, (static_cast<int64_t>(rows_a - 1) * lda + K) * 2);
+  const __amdgpu_buffer_rsrc_t rb =
+      rsrc(B + static_cast<int64_t>(n0) * ldb, (static_cast<int64_t>(rows_b - 1) * ldb + K) * 2);
+
+  const int kc = 8 * ((lane % 8) ^ (lane / 8));  // first column of this lane's 16 bytes in a slice (the swizzle)
+  unsigned offa[2][LA], offb[2][LB];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+#pragma unroll
+    for (int j = 0; j < LA; ++j) {
+      const int rr = 8 * (wave + j * NW) + lane / 8;
+      const int r = rr / QR * (2 * QR) + i * QR + rr % QR;
+      offa[i][j] = rr < 8 * kGroupsA && r < rows_a ? static_cast<unsigned>(r * lda * 2 + 2 * kc) : kNowhere;
+    }
+#pragma unroll
+    for (int j = 0; j < LB; ++j) {
+      const int rr = 8 * (wave + j * NW) + lane / 8;
+      const int r = rr / QC * (2 * QC) + i * QC + rr % QC;
+      offb[i][j] = rr < 8 * kGroupsB && r < rows_b ? static_cast<unsigned>(r * ldb * 2 + 2 * kc) : kNowhere;
+    }
+  }
+  const int ktiles = (ke - kb + kDmaBK - 1) / kDmaBK;
+  const int full = (ke - kb) / kDmaBK;
+  const KWalk walk(kb, ktiles, full == ktiles ? tn * rot_step : 0);
+  // The loads of half `i` of the slice at column k0 into buffer `buf`. Checked:
+  // also for slices that end past the K range (or start there: nothing is moved).
+  auto issue_a = [&](bool checked, int k0, int buf, int i) {
+    u32x4* base = lds + buf * kSlice + i * kHalfA;
+    const bool in = k0 + kc < ke;
+#pragma unroll
+    for (int j = 0; j < LA; ++j) {
+      const int off = static_cast<int>(checked ? (in ? offa[i][j] + 2 * k0 : kNowhere) : offa[i][j]);
+      u32x4* to = wave + j * NW < kGroupsA ? base + (wave + j * NW) * 64 : lds + 2 * kSlice;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (__attribute__((address_space(3))) void*)to, 16, off,
+                                               checked ? 0 : 2 * k0, 0, 0);
+    }
+  };
+  auto issue_b = [&](bool checked, int k0, int buf, int i) {
+    u32x4* base = lds + buf * kSlice + 2 * kHalfA + i * kHalfB;
+    const bool in = k0 + kc < ke;
+#pragma unroll
+    for (int j = 0; j < LB; ++j) {
+      const int off = static_cast<int>(checked ? (in ? offb[i][j] + 2 * k0 : kNowhere) : offb[i][j]);
+      u32x4* to = wave + j * NW < kGroupsB ? base + (wave + j * NW) * 64 : lds + 2 * kSlice;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (__attribute__((address_space(3))) void*)to, 16, off,
+                                               checked ? 0 : 2 * k0, 0, 0);
+    }
+  };
+
+  const int fa = (wm * QR + l16) * 8 + (lg ^ (l16 & 7));
+  const int fb = (wn * QC + l16) * 8 + (lg ^ (l16 & 7));
+  auto read_a = [&](int buf, int i, u32x4 (&f)[QM][2]) {
+    const u32x4* base = lds + buf * kSlice + i * kHalfA;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int q = 0; q < QM; ++q) f[q][h] = base[(fa ^ (4 * h)) + 128 * q];
+  };
+  auto read_b = [&](int buf, int i, u32x4 (&f)[QN][2]) {
+    const u32x4* base = lds + buf * kSlice + 2 * kHalfA + i * kHalfB;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int q = 0; q < QN; ++q) f[q][h] = base[(fb ^ (4 * h)) + 128 * q];
+  };
+
+  f32x4 acc[2 * QM][2 * QN];
+#pragma unroll
+  for (int i = 0; i < 2 * QM; ++i)
+#pragma unroll
+    for (int j = 0; j < 2 * QN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  u32x4 af[QM][2], b1[QN][2], bx[QN][2], by[QN][2];
+
+  auto multiply = [&](int i, int j, const u32x4 (&b)[QN][2]) {
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int q = 0; q < QM; ++q)
+#pragma unroll
+        for (int r = 0; r < QN; ++r)
+          acc[i * QM + q][j * QN + r] = E::mfma_16x16x32(b[r][h], af[q][h], acc[i * QM + q][j * QN + r]);
+    __builtin_amdgcn_s_setprio(0);
+  };
+
+  // Six of a slice's eight half loads stay in flight (see above).
+  auto mem_done = [&]() { pp_wait_barrier<3 * (LA + LB)>(); };
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    issue_b(true, walk.at(s), s, 0);
+    issue_a(true, walk.at(s), s, 0);
+    issue_b(true, walk.at(s), s, 1);
+    issue_a(true, walk.at(s), s, 1);
+  }
+  mem_done();  // halves B0 and A0 of slice 0 are in LDS
+  read_b(0, 0, bx);
+  mem_done();
+  if (wave >= NW / 2) pp_barrier();
+
+  // One K slice from buffer `buf`, which the slice at column k0 refills; b0
+  // holds its B0 fragments, those of the next slice go to bn.
+  auto slice = [&](bool checked, int k0, int buf, const u32x4 (&b0)[QN][2], u32x4 (&bn)[QN][2]) {
+    read_a(buf, 0, af);
+    issue_b(checked, k0, buf, 0);
+    mem_done();
+    multiply(0, 0, b0);
+    pp_barrier();
+    read_b(buf, 1, b1);
+    issue_a(checked, k0, buf, 0);
+    mem_done();
+    multiply(0, 1, b1);
+    pp_barrier();
+    read_a(buf, 1, af);
+    issue_b(checked, k0, buf, 1);
+    mem_done();
+    multiply(1, 1, b1);
+    pp_barrier();
+    read_b(buf ^ 1, 0, bn);
+    issue_a(checked, k0, buf, 1);
+    mem_done();
+    multiply(1, 0, b0);
+    pp_barrier();
+  };
+  int t = 0;
+  int k0 = walk.at(2);
+  for (; t + 3 < full; t += 2) {
+    slice(false, k0, 0, bx, by);
+    k0 = walk.after(k0);
+    slice(false, k0, 1, by, bx);
+    k0 = walk.after(k0);
+  }
+  for (; t < ktiles; t += 2) {
+    slice(true, walk.at(t + 2), 0, bx, by);
+    if (t + 1 < ktiles) slice(true, walk.at(t + 3), 1, by, bx);
+  }
+  if (wave < NW / 2) pp_barrier();
+
+  // The loads issued past the last slice move no data, but none may still be
+  // in flight into this workgroup's LDS when it is used again.
+  __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));
+  store_tile<E, 2 * QM, 2 * QN>(acc, lds, lane, wave, m0 + wm * 2 * QR, n0 + wn * 2 * QC, bias, C, M, N, ldc, vec_store,
+                                part);
+}
+
+// 2-stage tiles whose halves split into 16-row and 16-column fragments for 8
+// waves run the ping-pong body (256 x 256, 256 x 192; not 256 x 224 and
+// 192 x 224), the others the ring.
+template <int BN, int STAGES>
+constexpr bool ping_pong() {
+  return STAGES == 2 && BN % 64 == 0;
+}
+
+// Two waves per SIMD as the register target, also where the LDS allows one: with
+// the whole register file the compiler keeps the sums of the 4-wave tiles in
+// accumulation registers and moves them back and forth each slice (64 x 64: 36
+// ns a slice, 5.6 -> 6.1 us at N = K = 896).
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Wpass-failed"
+template <typename E, int BM, int BN, int WM, int WN, int STAGES>
+__global__ __launch_bounds__(WM * WN * kWave, 2) void gemm_dma_kernel(const uint16_t* __restrict__ A,
+                                                                   const uint16_t* __restrict__ B,
+                                                                   const uint16_t* __restrict__ bias,
+                                                                   uint16_t* __restrict__ C, int M, int N, int K,
+                                                                   int lda, int ldb, int ldc, int vec_store,
+                                                                   float* __restrict__ part, int k_split, int rot_step) {
+  if constexpr (ping_pong<BN, STAGES>())
+    ping_pong_tile<E, BM, BN, WM, WN>(A, B, bias, C, M, N, K, lda, ldb, ldc, vec_store, part, k_split, rot_step);
+  else
+    ring_tile<E, BM, BN, WM, WN, STAGES>(A, B, bias, C, M, N, K, lda, ldb, ldc, vec_store, part, k_split, rot_step);
+}
+#pragma clang diagnostic pop
 
 // With part != nullptr the K splits write fp32 partial tiles; `reduce` then
 // launches gemm_splitk_reduce_kernel, otherwise the caller consumes them.
 template <typename E, int BM, int BN, int WM, int WN, int STAGES>
 hipError_t launch_dma(const uint16_t* A, const uint16_t* B, const uint16_t* bias, uint16_t* C, int M, int N, int K,
-                      int lda, int ldb, int ldc, hipStream_t s, float* part, int splits, int k_split, bool reduce) {
+                      int lda, int ldb, int ldc, hipStream_t s, float* part, int splits, int k_split, bool reduce, int rot_step) {
   const int64_t tiles = ceil_div64(M, BM) * ceil_div64(N, BN);
   // Output stores of 16 bytes, or 8 where C's rows allow only that.
   const int vec = (ldc % 8 == 0 && aligned_to(C, 16)) ? 2 : (ldc % 4 == 0 && aligned_to(C, 8)) ? 1 : 0;
   hipLaunchKernelGGL((gemm_dma_kernel<E, BM, BN, WM, WN, STAGES>),
                      dim3(static_cast<unsigned>(tiles), static_cast<unsigned>(part != nullptr ? splits : 1)),
                      dim3(WM * WN * kWave), 0, s, A, B, bias, C, M, N, K, lda, ldb, ldc, vec, part,
-                     part != nullptr ? k_split : K);
+                     part != nullptr ? k_split : K, rot_step);
   if (part == nullptr || !reduce) return hipGetLastError();
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
@@ -635,7 +971,7 @@ hipError_t launch_dma(const uint16_t* A, const uint16_t* B, const uint16_t* bias
 }
 
 using DmaLauncher = hipError_t (*)(const uint16_t*, const uint16_t*, const uint16_t*, uint16_t*, int, int, int, int,
-                                   int, int, hipStream_t, float*, int, int, bool);
+                                   int, int, hipStream_t, float*, int, int, bool, int);
 
 // Launchers of kDmaShapes' tile shapes, in the same order.
 template <typename E>
@@ -875,6 +1211,17 @@ inline int64_t dma_workspace_bytes(const DmaPlan& d, int M, int N) {
   return d.splits > 1 ? static_cast<int64_t>(d.splits) * M * N * static_cast<int64_t>(sizeof(float)) : 0;
 }
 
+// K-walk rotation (see gemm_skinny_lds_kernel): column tile j starts its walk
+// j slices in. With one tile row every weight byte is read by one workgroup,
+// and spreading the walks spreads the reads over the HBM channels where rows
+// are 8 KB or 16 KB apart: gate_up (N 28672, K 4096) at M = 64 / 128 / 250
+// 52.4 / 57.8 / 69.5 -> 42.2 / 50.0 / 62.5 us, N = 128256 at M = 16 219 -> 176;
+// at K = 3584 and 5120 within 1%. With more tile rows, whose workgroups share
+// weight rows, and below 128 workgroups it measured 0-4% slower.
+inline int rotation(int64_t tiles_m, int64_t tiles_n, int splits) {
+  return splits == 1 && tiles_m == 1 && tiles_n >= 128 ? 1 : 0;
+}
+
 // The LDS-DMA kernel at decode sizes (M <= 64), on one 64-row tile: column
 // tiles of bn = 64 (4 waves, two workgroups per CU) or 128 (4 waves, one per
 // CU), K split over workgroup rows. Where it applies it replaces the skinny
@@ -970,7 +1317,7 @@ hipError_t launch(const uint16_t* A, const uint16_t* B, const uint16_t* bias, ui
       if (deferred_splits != nullptr) *deferred_splits = d.splits;
       const DmaLauncher fn = d.bn == 64 ? launch_dma<E, 64, 64, 2, 2, 4> : launch_dma<E, 64, 128, 2, 2, 4>;
       return fn(A, B, bias, C, M, N, K, lda, ldb, ldc, s, d.splits > 1 ? static_cast<float*>(workspace) : nullptr,
-                d.splits, d.k_split, deferred_splits == nullptr);
+                d.splits, d.k_split, deferred_splits == nullptr, rotation(1, ceil_div64(N, d.bn), d.splits));
     }
     float* part = p.splits > 1 ? static_cast<float*>(workspace) : nullptr;
     if (deferred_splits != nullptr) *deferred_splits = p.splits;
@@ -1004,7 +1351,9 @@ hipError_t launch(const uint16_t* A, const uint16_t* B, const uint16_t* bias, ui
   if (deferred_splits != nullptr) *deferred_splits = u.splits;
   return dma_launchers<E>()[u.shape](A, B, bias, C, M, N, K, lda, ldb, ldc, s,
                                      split ? static_cast<float*>(workspace) : nullptr, u.splits, u.k_split,
-                                     deferred_splits == nullptr);
+                                     deferred_splits == nullptr,
+                                     rotation(ceil_div64(M, kDmaShapes[u.shape].bm),
+                                              ceil_div64(N, kDmaShapes[u.shape].bn), u.splits));
 }
 
 }  // namespace gemm
