@@ -234,6 +234,17 @@ def gemm_plan(M: int, N: int, K: int, with_workspace: bool = True) -> tuple[int,
     return tuple(out)
 
 
+def gemm_tile(M: int, N: int, K: int, with_workspace: bool = True) -> tuple[int, int, int, int]:
+    """What runs gemm_tn's plan for this shape; host arithmetic only: (tile
+    rows, tile columns, K splits, K-walk rotation) of the tiled kernel, or the
+    skinny kernel's (waves along N, waves along K, K splits, 0)."""
+    out = (ctypes.c_int * 4)()
+    rc = lib().dk_gemm_tn_tile(M, N, K, int(with_workspace), out)
+    if rc != 0:
+        raise ValueError(last_error())
+    return tuple(out)
+
+
 def last_error() -> str:
     return lib().dk_last_error().decode()
 

@@ -21,12 +21,14 @@
 //   in flight across the per-step barrier.
 // * LDS-DMA (M > 64, batched decode and prefill): A and B tiles go from HBM
 //   straight into LDS (buffer_load ... lds), bank-conflict-free XOR-swizzled,
-//   through a multi-stage ring; nine tile shapes from 256x256 down to 64x64,
-//   picked per call by a throughput model so that batches of a few hundred
+//   through a multi-stage ring; thirteen tile shapes from 256x256 down to 64x64.
+//   A plan per size sets the workspace and the most K splits; a time model
+//   picks the tile that runs it (kTileModel), so that batches of a few hundred
 //   rows still fill all 256 CUs. The output tile leaves through the freed
 //   ring, read back row by row for 16-byte stores. At M <= 64 its 64-row
 //   tiles (64 or 128 columns, K split) replace the skinny kernel from M = 32
-//   where they fill the CUs, and for N > 32768 (decode_dma_plan).
+//   where they fill the CUs, for N > 32768 (decode_dma_plan), and where they
+//   measured faster at any M (decode_tile_plan).
 #include <algorithm>
 
 #include "../../include/decodekernels_amd.h"
@@ -924,8 +926,8 @@ __device__ __forceinline__ void ping_pong_tile(const uint16_t* __restrict__ A, c
 }
 
 // 2-stage tiles whose halves split into 16-row and 16-column fragments for 8
-// waves run the ping-pong body (256 x 256, 256 x 192; not 256 x 224 and
-// 192 x 224), the others the ring.
+// waves run the ping-pong body (256 x 256, 256 x 192, 192 x 256, 256 x 128,
+// 128 x 256; not 256 x 224 and 192 x 224), the others the ring.
 template <int BN, int STAGES>
 constexpr bool ping_pong() {
   return STAGES == 2 && BN % 64 == 0;
@@ -973,13 +975,15 @@ hipError_t launch_dma(const uint16_t* A, const uint16_t* B, const uint16_t* bias
 using DmaLauncher = hipError_t (*)(const uint16_t*, const uint16_t*, const uint16_t*, uint16_t*, int, int, int, int,
                                    int, int, hipStream_t, float*, int, int, bool, int);
 
-// Launchers of kDmaShapes' tile shapes, in the same order.
+// Launchers of kTileShapes' tile shapes, in the same order.
 template <typename E>
-const DmaLauncher* dma_launchers() {
+const DmaLauncher* tile_launchers() {
   static const DmaLauncher fns[] = {
-      launch_dma<E, 256, 256, 4, 2, 2>, launch_dma<E, 256, 224, 4, 2, 2>, launch_dma<E, 256, 192, 4, 2, 2>,
-      launch_dma<E, 256, 128, 4, 2, 3>, launch_dma<E, 192, 224, 4, 2, 2>, launch_dma<E, 192, 192, 4, 2, 3>,
-      launch_dma<E, 128, 128, 4, 2, 3>, launch_dma<E, 128, 64, 2, 2, 4>,  launch_dma<E, 64, 64, 2, 2, 4>,
+      launch_dma<E, 256, 256, 4, 2, 2>, launch_dma<E, 256, 192, 4, 2, 2>, launch_dma<E, 192, 256, 2, 4, 2>,
+      launch_dma<E, 256, 128, 4, 2, 2>, launch_dma<E, 128, 256, 2, 4, 2>, launch_dma<E, 128, 128, 4, 2, 3>,
+      launch_dma<E, 128, 160, 4, 2, 4>, launch_dma<E, 128, 64, 2, 2, 4>,  launch_dma<E, 64, 64, 2, 2, 4>,
+      launch_dma<E, 64, 128, 2, 2, 4>,  launch_dma<E, 192, 192, 4, 2, 3>, launch_dma<E, 192, 224, 4, 2, 2>,
+      launch_dma<E, 256, 224, 4, 2, 2>,
   };
   return fns;
 }
@@ -1211,6 +1215,57 @@ inline int64_t dma_workspace_bytes(const DmaPlan& d, int M, int N) {
   return d.splits > 1 ? static_cast<int64_t>(d.splits) * M * N * static_cast<int64_t>(sizeof(float)) : 0;
 }
 
+// Tile that runs a plan: of the shapes, with at most the plan's K splits -- so
+// its workspace holds them, and an unsplit plan stays unsplit and gives the
+// same bits with and without a workspace -- the one with the smallest modelled
+// time. Microseconds, with n slices of 64 columns per split and W workgroups:
+//   start + n x slice x rounds + tile x ceil(W / 256)
+//     + [split] (split + per_split x splits + splits x M x N x 8 B / partials),
+// joined as (t^4 + m^4)^(1/4) with the time m of the operands and the output
+// at `memory` bytes a microsecond. A part-filled round of 256 workgroups takes
+// part_fill to 1 of a full one (its workgroups get more of the memory), times
+// last_round behind full ones. The 64 x 64 tile is paced by the latency of a
+// slice: each of its rounds counts whole (0.20 / 0.36 / 0.56 us a slice with 1 /
+// 2 / 3 workgroups to a CU, however many CUs have them).
+struct TileModel {
+  double start, split, per_split, partials, memory, part_fill, last_round;
+};
+struct TileShape {
+  int bm, bn;
+  double slice_us, tile_us;
+  bool whole_rounds;
+};
+struct TilePlan {
+  int shape, splits, k_split, rot_step;
+};
+
+// M > 64. Fitted to 250 (M, N, K) of the Llama-3-8B, Qwen2.5-7B and
+// Qwen2.5-0.5B projections and fifteen other (N, K), M = 65 ... 4096, every
+// shape with 1, 2, 3, 4, 6 and 8 splits, calls on three sets of operands in
+// turn: the pick is 0.6% slower than the fastest choice on average (worst 24%,
+// N 10387, K 624) and 1.35x faster than hipBLASLt (geometric means). Against
+// the plan's own tile in the ring body (us): qkv_proj of Qwen2.5-7B (N 4608,
+// K 3584) at M = 1003 47.5 -> 36.9, Llama-3-8B gate_up at M = 1003 201 -> 178,
+// down at M = 1003 / 2048 118 / 215 -> 101 / 175.
+constexpr TileModel kTileModel{2.61, 1.42, 0.234, 7.27e6, 4.99e6, 0.62, 1.148};
+constexpr TileShape kTileShapes[] = {
+    {256, 256, 1.233, 5.10, false}, {256, 192, 1.026, 6.34, false}, {192, 256, 0.993, 5.64, false},
+    {256, 128, 0.820, 3.59, false}, {128, 256, 0.821, 4.25, false}, {128, 128, 0.516, 1.51, false},
+    {128, 160, 0.622, 2.77, false}, {128, 64, 0.344, 1.54, false}, {64, 64, 0.184, 0.83, true},
+    {64, 128, 0.368, 2.00, false}, {192, 192, 0.900, 6.00, false}, {192, 224, 1.134, 6.20, false},
+    {256, 224, 1.415, 5.91, false},
+};
+constexpr int kTileCount = static_cast<int>(sizeof(kTileShapes) / sizeof(kTileShapes[0]));
+constexpr int kTile64x64 = 8, kTile64x128 = 9;  // their places in kTileShapes
+
+// M <= 64, plans of three splits or more. Fitted to 57 (M, N, K), M = 1 ... 64:
+// 1.0% slower than the fastest choice on average, 9% faster than the plan's
+// own kernel (worst 8% slower: N 3584, K 18944 at M = 64, 30.0 -> 32.5). Llama-3-8B at M = 64: qkv 15.0 (64 x
+// 128, 4 splits) -> 13.6 us (64 x 64, 2); Qwen2.5-7B qkv at M = 1 / 64 11.2 / 13.1
+// -> 9.2 / 11.3; N 3072, K 8192 at M = 64 15.3 -> 13.7.
+constexpr TileModel kDecodeModel{2.4, 1.672, 0.222, 8.24e6, 6.393e6, 0.636, 1.0};
+constexpr TileShape kDecodeShapes[] = {{64, 64, 0.207, 0.519, true}, {64, 128, 0.370, 1.027, false}};
+
 // K-walk rotation (see gemm_skinny_lds_kernel): column tile j starts its walk
 // j slices in. With one tile row every weight byte is read by one workgroup,
 // and spreading the walks spreads the reads over the HBM channels where rows
@@ -1220,6 +1275,50 @@ inline int64_t dma_workspace_bytes(const DmaPlan& d, int M, int N) {
 // weight rows, and below 128 workgroups it measured 0-4% slower.
 inline int rotation(int64_t tiles_m, int64_t tiles_n, int splits) {
   return splits == 1 && tiles_m == 1 && tiles_n >= 128 ? 1 : 0;
+}
+
+inline TilePlan fastest_tile(const TileModel& m, const TileShape* shapes, int count, int M, int N, int K,
+                             int max_splits) {
+  TilePlan best{0, 1, K, 0};
+  double best_t = -1.0;
+  const double mn = static_cast<double>(M) * N;
+  const double mem = 2.0 * (static_cast<double>(M) * K + static_cast<double>(N) * K + mn) / m.memory;
+  const double mem4 = mem * mem * mem * mem;
+  for (int i = 0; i < count; ++i) {
+    const TileShape& sh = shapes[i];
+    const int64_t tiles_m = ceil_div64(M, sh.bm);
+    const int64_t tiles_n = ceil_div64(N, sh.bn);
+    for (const int s : {1, 2, 3, 4, 6, 8}) {
+      int ks = K;
+      if (s > 1) {
+        if (s > max_splits || tiles_m * tiles_n > kSkinnyCus || K / s < 512) break;
+        ks = ((K + s - 1) / s + kDmaBK - 1) / kDmaBK * kDmaBK;
+        if ((K + ks - 1) / ks != s) continue;  // every split non-empty
+      }
+      const int64_t wgs = tiles_m * tiles_n * s;
+      const double n = static_cast<double>((ks + kDmaBK - 1) / kDmaBK);
+      const int64_t full = wgs / kSkinnyCus;
+      const int64_t rem = wgs % kSkinnyCus;
+      double rounds = static_cast<double>(full);
+      if (rem > 0) {
+        const double part =
+            sh.whole_rounds ? 1.0 : m.part_fill + (1.0 - m.part_fill) * static_cast<double>(rem) / kSkinnyCus;
+        rounds += (full > 0 && !sh.whole_rounds ? m.last_round : 1.0) * part;
+      }
+      double t = m.start + n * sh.slice_us * rounds + sh.tile_us * static_cast<double>(full + (rem > 0 ? 1 : 0));
+      if (s > 1) t += m.split + m.per_split * s + s * mn * 8.0 / m.partials;
+      t = t * t * t * t + mem4;
+      if (best_t < 0 || t < best_t) {
+        best = TilePlan{i, s, ks, rotation(tiles_m, tiles_n, s)};
+        best_t = t;
+      }
+    }
+  }
+  return best;
+}
+
+inline TilePlan tile_plan(int M, int N, int K, int plan_splits) {
+  return fastest_tile(kTileModel, kTileShapes, kTileCount, M, N, K, plan_splits);
 }
 
 // The LDS-DMA kernel at decode sizes (M <= 64), on one 64-row tile: column
@@ -1292,6 +1391,80 @@ inline int64_t decode_dma_workspace_bytes(const DecodeDmaPlan& d, int M, int N) 
   return d.bn > 0 && d.splits > 1 ? static_cast<int64_t>(d.splits) * M * N * static_cast<int64_t>(sizeof(float)) : 0;
 }
 
+// Tile that runs a decode plan (M <= 64) in place of its kernel; shape < 0:
+// none. Plans of three splits or more go to the faster of the two 64-row tiles
+// (kDecodeModel). Unsplit, a wide weight matrix is read fastest by 64-row
+// tiles with the K walks rotated; the lines are where the tiles fill the chip
+// (us, the plan's own kernel -> the tile, calls on three sets of operands in
+// turn; K < 2048 was not measured):
+//  * 64 x 64 when it has 192 to 256 tiles (two to a CU), over any plan: N 12288
+//    / 14336 / 16384 (K 4096) at M = 1 20.1 / 21.8 / 27.3 -> 17.5 / 20.5 / 24.4,
+//    at M = 64 24.4 / 29.8 / 35.3 -> 20.4 / 24.0 / 26.0; N 12288, K 6144 at M = 1
+//    29.3 against 29.9;
+//  * 64 x 128 when its last round fills 3/4 of the 256 CUs, over an unsplit
+//    plan: gate_up (N 28672, K 4096) M = 1 / 16 / 64 41.6 / 41.4 / 48.7 -> 39.5 /
+//    40.1 / 42.5, N 24576 at M = 1 35.9 -> 33.5, N 128256 at M = 1 / 16 / 64 194 /
+//    199 / 220 -> 171 / 176 / 182, N 57344 (K 8192) 169 -> 157. Below: N 20480
+//    (160 tiles, K 5120) 37.6 against 39.1, N 37888 (296) 52.7 against 60.
+inline TilePlan decode_tile_plan(int M, int N, int K, int plan_splits) {
+  const int64_t t128 = ceil_div64(N, 128);
+  const int64_t t64 = ceil_div64(N, 64);
+  if (K >= 2048 && t64 >= 192 && t64 <= kSkinnyCus) return TilePlan{kTile64x64, 1, K, rotation(1, t64, 1)};
+  if (K >= 2048 && plan_splits == 1 && t64 > kSkinnyCus &&
+      4 * t128 >= 3 * kSkinnyCus * ceil_div64(t128, kSkinnyCus))
+    return TilePlan{kTile64x128, 1, K, rotation(1, t128, 1)};
+  if (plan_splits < 3) return TilePlan{-1, 1, K, 0};
+  TilePlan t = fastest_tile(kDecodeModel, kDecodeShapes, 2, M, N, K, plan_splits);
+  t.shape = t.shape == 0 ? kTile64x64 : kTile64x128;
+  // At small M the skinny kernel's 5-6% lead at short K (us: N 5731, K 5496, M = 1
+  // 16.0 against 17.1; N 8765, K 5608, M = 2 22.8 against 24.3) turns with K (N
+  // 10240, K 8192, M = 1 39.0 against 32.5).
+  if (t.shape == kTile64x128 && M < 32 && K < 8192) return TilePlan{-1, 1, K, 0};
+  // Below half of the CUs the skinny kernel's narrower tiles read faster (N 896,
+  // K 4864, M = 6: 6.8 us against 8.8 with 56 workgroups).
+  return ceil_div64(N, kTileShapes[t.shape].bn) * t.splits >= kSkinnyCus / 2 ? t : TilePlan{-1, 1, K, 0};
+}
+
+// What a call of one size runs with a full workspace: the plan, the tile that
+// runs it, and the plan's workspace. A function of the sizes alone, kept per
+// thread in a small direct-mapped table: a call asks for it twice (workspace,
+// launch), and its evaluation (0.3-1 us of host time) shows where the kernel
+// takes less than its launch.
+struct CallPlan {
+  int M, N, K;  // M = 0: an empty entry
+  int64_t workspace_bytes;
+  DmaPlan dma;             // M > 64
+  DecodeDmaPlan decode;    // M <= 64, and
+  SkinnyPlan skinny;       // where decode.bn = 0
+  TilePlan tile;
+};
+
+inline CallPlan make_call_plan(int M, int N, int K) {
+  CallPlan c{M, N, K, 0, {}, {}, {}, {}};
+  if (M > 64) {
+    c.dma = dma_plan(M, N, K, true);
+    c.workspace_bytes = dma_workspace_bytes(c.dma, M, N);
+    c.tile = tile_plan(M, N, K, c.dma.splits);
+  } else {
+    c.decode = decode_dma_plan(M, N, K, true);
+    c.skinny = skinny_plan(M, N, K, true);
+    c.workspace_bytes =
+        c.decode.bn > 0 ? decode_dma_workspace_bytes(c.decode, M, N) : skinny_workspace_bytes(c.skinny, M, N);
+    c.tile = decode_tile_plan(M, N, K, c.decode.bn > 0 ? c.decode.splits : c.skinny.splits);
+  }
+  return c;
+}
+
+inline const CallPlan& call_plan(int M, int N, int K) {
+  constexpr unsigned kEntries = 64;
+  static thread_local CallPlan table[kEntries];
+  const unsigned h = static_cast<unsigned>(M) * 0x9E3779B1u ^ static_cast<unsigned>(N) * 0x85EBCA77u ^
+                     static_cast<unsigned>(K) * 0xC2B2AE3Du;
+  CallPlan& c = table[(h >> 16) % kEntries];
+  if (c.M != M || c.N != N || c.K != K) c = make_call_plan(M, N, K);
+  return c;
+}
+
 // Launches C = A B^T (+ bias) with the plan for (M, N, K) and the workspace
 // given. With deferred_splits != nullptr, a plan that splits K stops after the
 // main kernel, leaving splits x M x N fp32 partial tiles (no bias) in the
@@ -1303,21 +1476,30 @@ hipError_t launch(const uint16_t* A, const uint16_t* B, const uint16_t* bias, ui
                   int lda, int ldb, int ldc, void* workspace, int64_t workspace_bytes, hipStream_t s,
                   int* deferred_splits, bool dma_ok) {
   if (M <= 64) {
-    constexpr DecodeDmaPlan kNone{0, 1, 0};
-    DecodeDmaPlan d = dma_ok ? decode_dma_plan(M, N, K, true) : kNone;
-    SkinnyPlan p = skinny_plan(M, N, K, true);
+    const CallPlan& full = call_plan(M, N, K);
+    DecodeDmaPlan d = dma_ok ? full.decode : DecodeDmaPlan{0, 1, 0};
+    SkinnyPlan p = full.skinny;
+    TilePlan t = full.tile;
     // A workspace smaller than the plan's needs runs exactly the plan
     // without one (both kernels' choices then exclude splits).
     const int64_t need = d.bn > 0 ? decode_dma_workspace_bytes(d, M, N) : skinny_workspace_bytes(p, M, N);
     if (need > 0 && (workspace == nullptr || need > workspace_bytes)) {
-      d = dma_ok ? decode_dma_plan(M, N, K, false) : kNone;
+      if (dma_ok) d = decode_dma_plan(M, N, K, false);
       p = skinny_plan(M, N, K, false);
+      t = decode_tile_plan(M, N, K, 1);
+    }
+    if (!dma_ok) t.shape = -1;
+    if (t.shape >= 0) {
+      if (deferred_splits != nullptr) *deferred_splits = t.splits;
+      return tile_launchers<E>()[t.shape](A, B, bias, C, M, N, K, lda, ldb, ldc, s,
+                                          t.splits > 1 ? static_cast<float*>(workspace) : nullptr, t.splits, t.k_split,
+                                          deferred_splits == nullptr, t.rot_step);
     }
     if (d.bn > 0) {
       if (deferred_splits != nullptr) *deferred_splits = d.splits;
-      const DmaLauncher fn = d.bn == 64 ? launch_dma<E, 64, 64, 2, 2, 4> : launch_dma<E, 64, 128, 2, 2, 4>;
-      return fn(A, B, bias, C, M, N, K, lda, ldb, ldc, s, d.splits > 1 ? static_cast<float*>(workspace) : nullptr,
-                d.splits, d.k_split, deferred_splits == nullptr, rotation(1, ceil_div64(N, d.bn), d.splits));
+      return tile_launchers<E>()[d.bn == 64 ? kTile64x64 : kTile64x128](
+          A, B, bias, C, M, N, K, lda, ldb, ldc, s, d.splits > 1 ? static_cast<float*>(workspace) : nullptr, d.splits,
+          d.k_split, deferred_splits == nullptr, rotation(1, ceil_div64(N, d.bn), d.splits));
     }
     float* part = p.splits > 1 ? static_cast<float*>(workspace) : nullptr;
     if (deferred_splits != nullptr) *deferred_splits = p.splits;
@@ -1345,15 +1527,13 @@ hipError_t launch(const uint16_t* A, const uint16_t* B, const uint16_t* bias, ui
     }
     return hipGetLastError();
   }
-  const DmaPlan d = dma_plan(M, N, K, workspace != nullptr);
-  const bool split = d.splits > 1 && dma_workspace_bytes(d, M, N) <= workspace_bytes;
-  const DmaPlan u = split ? d : dma_plan(M, N, K, false);
-  if (deferred_splits != nullptr) *deferred_splits = u.splits;
-  return dma_launchers<E>()[u.shape](A, B, bias, C, M, N, K, lda, ldb, ldc, s,
-                                     split ? static_cast<float*>(workspace) : nullptr, u.splits, u.k_split,
-                                     deferred_splits == nullptr,
-                                     rotation(ceil_div64(M, kDmaShapes[u.shape].bm),
-                                              ceil_div64(N, kDmaShapes[u.shape].bn), u.splits));
+  const CallPlan& full = call_plan(M, N, K);
+  const bool fits = full.workspace_bytes == 0 || (workspace != nullptr && full.workspace_bytes <= workspace_bytes);
+  const TilePlan t = fits ? full.tile : tile_plan(M, N, K, 1);
+  if (deferred_splits != nullptr) *deferred_splits = t.splits;
+  return tile_launchers<E>()[t.shape](A, B, bias, C, M, N, K, lda, ldb, ldc, s,
+                                      t.splits > 1 ? static_cast<float*>(workspace) : nullptr, t.splits, t.k_split,
+                                      deferred_splits == nullptr, t.rot_step);
 }
 
 }  // namespace gemm
@@ -1414,11 +1594,7 @@ extern "C" int dk_gemm_tn(int dtype, const void* A, const void* B, const void* b
 
 extern "C" int64_t dk_gemm_tn_workspace_bytes(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  if (M > 64) return dk::gemm::dma_workspace_bytes(dk::gemm::dma_plan(M, N, K, true), M, N);
-  const dk::gemm::DecodeDmaPlan d = dk::gemm::decode_dma_plan(M, N, K, true);
-  if (d.bn > 0) return dk::gemm::decode_dma_workspace_bytes(d, M, N);
-  const dk::gemm::SkinnyPlan p = dk::gemm::skinny_plan(M, N, K, true);
-  return dk::gemm::skinny_workspace_bytes(p, M, N);
+  return dk::gemm::call_plan(M, N, K).workspace_bytes;
 }
 
 extern "C" int dk_gemm_tn_plan(int M, int N, int K, int with_workspace, int* plan) {
@@ -1446,6 +1622,27 @@ extern "C" int dk_gemm_tn_plan(int M, int N, int K, int with_workspace, int* pla
   plan[1] = p.wk;
   plan[2] = p.splits;
   plan[3] = p.k_split;
+  return hipSuccess;
+}
+
+extern "C" int dk_gemm_tn_tile(int M, int N, int K, int with_workspace, int* tile) {
+  using namespace dk;
+  using namespace dk::gemm;
+  int plan[4];
+  if (tile == nullptr) return fail("gemm_tn_tile: tile must not be NULL");
+  if (const int rc = dk_gemm_tn_plan(M, N, K, with_workspace, plan)) return rc;
+  const TilePlan t = M > 64 ? tile_plan(M, N, K, plan[2]) : decode_tile_plan(M, N, K, plan[2]);
+  if (t.shape >= 0) {
+    tile[0] = kTileShapes[t.shape].bm;
+    tile[1] = kTileShapes[t.shape].bn;
+    tile[2] = t.splits;
+    tile[3] = t.rot_step;
+  } else {
+    tile[0] = plan[0];
+    tile[1] = plan[1];
+    tile[2] = plan[2];
+    tile[3] = plan[0] == 64 ? rotation(1, ceil_div64(N, plan[1]), plan[2]) : 0;
+  }
   return hipSuccess;
 }
 

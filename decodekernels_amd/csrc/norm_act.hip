@@ -328,7 +328,9 @@ void launch_splitk_add_nv(uint16_t* out, uint16_t* r, const uint16_t* w, int row
     return;
   switch (splits) {
     DK_SPLIT_CASE(2)
+    DK_SPLIT_CASE(3)
     DK_SPLIT_CASE(4)
+    DK_SPLIT_CASE(6)
     DK_SPLIT_CASE(8)
     default:
       hipLaunchKernelGGL((splitk_add_rms_norm_kernel<E, NV, 0>), dim3(rows), block, 0, s, out, r, w, H, os, rs_, eps,

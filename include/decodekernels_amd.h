@@ -148,10 +148,20 @@ int64_t dk_gemm_tn_workspace_bytes(int M, int N, int K);
  * workgroup (16 columns each), waves along K, K splits, columns per split;
  * tiled kernel (M > 64, and M <= 64 where 64-row tiles fill the CUs better:
  * plan[0] = 64) = tile rows, tile columns, K splits, columns per split. For
- * tests and tuning; launches nothing.
+ * tests and tuning; launches nothing. The plan sets the workspace and the most
+ * K splits a call may use; dk_gemm_tn_tile says which tile runs it.
  * No counterpart in DecodeKernels.
  */
 int dk_gemm_tn_plan(int M, int N, int K, int with_workspace, int* plan);
+
+/*
+ * What runs a plan: tile[0..3] = tile rows, tile columns, K splits (at most the
+ * plan's) and K-walk rotation (slices of 64 columns per column tile) of the
+ * tiled kernel, or, where the skinny kernel runs, the plan's first three
+ * numbers and 0. For tests and tuning; launches nothing.
+ * No counterpart in DecodeKernels.
+ */
+int dk_gemm_tn_tile(int M, int N, int K, int with_workspace, int* tile);
 
 /*
  * dk_gemm_tn with a caller-provided workspace (16-byte aligned). Decode
