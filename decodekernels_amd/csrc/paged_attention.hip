@@ -138,6 +138,7 @@ struct KParams {
   int lockstep;    // balanced kernel: groups of num_kv_heads workgroups share one token range (grid % heads == 0)
   float scale_log2;  // softmax scale x log2(e) (x k_scale for an fp8 cache)
   float v_scale;     // multiplies the output (fp8 cache's v_scale; 1 otherwise)
+  int max_seq_len;   // host side: the caller's bound on the lengths, for the launch shape
 };
 
 
@@ -1252,10 +1253,53 @@ constexpr int waves_per_group() {
   return D > 128 ? DK_ATTN_WAVES_D256 : kWaves;
 }
 
+// Workgroups of `kernel` that fit on the current device at once (0 if unknown)
+// and per CU, cached per device in `cache`.
+int resident_workgroups(const void* kernel, int threads, std::atomic<int>* cache, int* per_cu_out) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 0;
+  // Packed (workgroups per CU) << 20 | CUs.
+  int v = cache[dev].load(std::memory_order_relaxed);
+  if (v <= 0) {
+    int per_cu = 0;
+    int cus = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, threads, 0) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || per_cu <= 0 ||
+        per_cu > 1023 || cus <= 0 || cus >= (1 << 20))
+      return 0;
+    v = (per_cu << 20) | cus;
+    cache[dev].store(v, std::memory_order_relaxed);
+  }
+  if (per_cu_out != nullptr) *per_cu_out = v >> 20;
+  return (v >> 20) * (v & 0xfffff);
+}
+
 // Launches the grid kernel (BALANCED = false, one workgroup per unit slot) or
 // the balanced kernel for KV pointers aligned to ALIGN bytes. With
 // `resident`, only reports how many balanced-kernel workgroups fit on the
-// current device at once (0 if unknown), cached per device.
+// current device at once (0 if unknown).
+//
+// A grid of units of at most 512 tokens (single pass, or one per workspace
+// row) that leaves the chip part-filled takes workgroups of twice the waves:
+// such a call is a chain of memory round trips, two tiles a wave each, and every
+// wave then has half the tiles. Where it pays, per class (us, NW waves -> 2 NW,
+// 16-bit / fp8 cache; 360 calls, 1 to 64 sequences of 40 to 8192 tokens):
+//   head_dim > 128: while the grid fits in one round, 5-60% faster. 16 heads on
+//     2 KV heads of 256, 512 tokens: 1 sequence 22.9 -> 16.3 / 21.8 -> 13.6, 16
+//     sequences 23.3 -> 17.0 / 22.1 -> 14.3; 16 x 4096 tokens 31.5 -> 30.1;
+//   head_dim <= 64: up to one workgroup for two CUs, 2-20% faster. 14 heads on
+//     2 of 64: 8 x 512 7.5 -> 6.2 / 7.2 -> 6.3, 2 x 8192 11.3 -> 10.1. One per CU: 5%
+//     slower to 2% faster, two per CU: 0-3% slower (64 x 130 on 8 KV heads 6.0 -> 6.5);
+//   between: up to one workgroup for 8 CUs, 0-13% faster. 32 heads on 8 of 128:
+//     1 x 1000 11.5 -> 10.2 / 11.0 -> 10.3. From 64 workgroups on -3% ... +5%: the
+//     CU's other waves, not the chain, then bound a wave's loads.
+// With one tile a wave or less there is no chain to halve, and the larger merge
+// shows (1 x 40 tokens, head_dim 128: 4.4 -> 4.6).
+template <int D>
+constexpr int wide_limit(int resident, int cus) {
+  return D > 128 ? resident : (D <= 64 ? cus / 2 : cus / 8);
+}
+
 template <typename E, int D, int ALIGN, bool SPLIT, bool BS16, bool BALANCED, bool KV8>
 hipError_t launch_kernel(const KParams& kp, unsigned grid, hipStream_t stream, int* resident = nullptr,
                          int* per_cu_out = nullptr) {
@@ -1264,28 +1308,21 @@ hipError_t launch_kernel(const KParams& kp, unsigned grid, hipStream_t stream, i
     const auto kernel = paged_attention_balanced_kernel<E, D, BS16, ALIGN, NW, KV8>;
     if (resident != nullptr) {
       static std::atomic<int> cache[kMaxDevices];
-      *resident = 0;
-      int dev = 0;
-      if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return hipSuccess;
-      // Packed (workgroups per CU) << 20 | CUs.
-      int v = cache[dev].load(std::memory_order_relaxed);
-      if (v <= 0) {
-        int per_cu = 0;
-        int cus = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kernel), NW * kWave, 0) !=
-                hipSuccess ||
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-            per_cu <= 0 || per_cu > 1023 || cus <= 0 || cus >= (1 << 20))
-          return hipSuccess;
-        v = (per_cu << 20) | cus;
-        cache[dev].store(v, std::memory_order_relaxed);
-      }
-      *resident = (v >> 20) * (v & 0xfffff);
-      if (per_cu_out != nullptr) *per_cu_out = v >> 20;
+      *resident = resident_workgroups(reinterpret_cast<const void*>(kernel), NW * kWave, cache, per_cu_out);
       return hipSuccess;
     }
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(NW * kWave), 0, stream, kp);
   } else {
+    if ((!SPLIT || kp.unit512) && kp.max_seq_len > NW * kTile) {
+      static std::atomic<int> cache[kMaxDevices];
+      const auto wide = paged_attention_kernel<E, D, SPLIT, BS16, ALIGN, 2 * NW, KV8>;
+      int per_cu = 0;
+      const int fit = resident_workgroups(reinterpret_cast<const void*>(wide), 2 * NW * kWave, cache, &per_cu);
+      if (fit > 0 && static_cast<int64_t>(grid) <= wide_limit<D>(fit, fit / per_cu)) {
+        hipLaunchKernelGGL(wide, dim3(grid), dim3(2 * NW * kWave), 0, stream, kp);
+        return hipGetLastError();
+      }
+    }
     hipLaunchKernelGGL((paged_attention_kernel<E, D, SPLIT, BS16, ALIGN, NW, KV8>), dim3(grid), dim3(NW * kWave), 0, stream,
                        kp);
   }
@@ -1548,6 +1585,7 @@ int paged_attention_entry(const dk_paged_attn_params* a, int dtype, int head_dim
   kp.num_units = split ? static_cast<int>(ceil_div64(a->max_partitions, 2)) : 1;
   kp.scale_log2 = a->scale * k_scale * kLog2e;
   kp.v_scale = v_scale;
+  kp.max_seq_len = max_seq_len;
   if (static_cast<int64_t>(a->num_seqs) * a->num_kv_heads * (std::max(kp.num_units, kp.max_partitions) + 1) >=
       (int64_t{1} << 31))
     return fail("paged_attention_decode: num_seqs x num_kv_heads x partitions is too large");
