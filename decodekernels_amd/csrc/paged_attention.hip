@@ -1073,8 +1073,9 @@ void paged_attention_balanced_kernel(const KParams p) {
 // WPH waves per query head, max(4, WPH) waves per workgroup. The (m_p, s_p)
 // pairs are uniform across a wave and each lane accumulates D/64 output
 // columns; with WPH > 1 the waves of a head take every WPH-th row and merge
-// through LDS. The op is latency-bound: WPH grows with the number of rows a
-// head merges (1 wave up to 8, 4 up to 63, 16 beyond; measured).
+// through LDS. A few heads are a chain of latencies, and WPH grows with the
+// number of rows a head merges; many heads are bound by the waves, most of them
+// without a row (launch_reduce_sized).
 template <int WPH>
 constexpr int reduce_waves() {
   return WPH > 4 ? WPH : 4;
@@ -1390,7 +1391,18 @@ void launch_reduce_sized(const KParams& kp, int num_seqs, hipStream_t stream) {
   // Rows a head merges at most.
   const int entries = PIECES ? kp.max_partitions : 2 + (kp.max_partitions - 1) / 2;
   if (entries <= 8) launch_reduce<D, 1, PIECES, E>(kp, num_seqs, stream);
-  else if (entries < 64) launch_reduce<D, 4, PIECES, E>(kp, num_seqs, stream);
+  // 1 wave up to 8 rows, 4 up to 63, 16 beyond (measured) while all heads' waves
+  // are resident at once: 512 heads of 16 waves are 8192, the chip's wave slots.
+  // From there on 16 waves come in rounds, nearly all of them idle: a length
+  // bound of 64 rows says little about the pieces of a balanced share. Whole
+  // calls, us, 16 -> 4 waves (one 32768-token sequence among short ones: the
+  // longest chain): 1024 heads of 256, 64 x 2048 tokens 74.0 -> 68.5, one long
+  // 54.1 -> 50.3; 4096 heads 187 -> 173; 1792 heads of 64 39.3 -> 33.9; 2048 heads
+  // of 128, 64 x 16384 691 -> 684, one long 60.1 -> 53.1. At 512 heads one long
+  // 49.8 -> 49.3 (256) and 24.8 -> 24.6 (128); below, 16 waves win there: 256
+  // heads of 256 48.2 against 48.7, 224 heads of 64 13.8 against 14.1.
+  else if (entries < 64 || (PIECES && static_cast<int64_t>(kp.num_q_heads) * num_seqs >= 512))
+    launch_reduce<D, 4, PIECES, E>(kp, num_seqs, stream);
   else launch_reduce<D, 16, PIECES, E>(kp, num_seqs, stream);
 }
 
