@@ -238,11 +238,11 @@ __global__ __launch_bounds__(kThreads) void reshape_and_cache_fp8_kernel(const K
 
 namespace rope_cache {
 
-// 1024 threads per token: with a GEMM's split-K partials to sum first (a
-// [tokens, N] row each, 64 tokens at decode batch 64, so only 64 workgroups),
-// the row's loads are spread over four times the threads of the rotary /
-// cache work alone; 256 threads took 10.9 us for the qkv row of Llama-3-8B at
-// batch 64, more than the separate reduce and rotary kernels together.
+// The largest workgroup, and the one taken where a GEMM's split-K partials are
+// summed first (a [tokens, N] row each, 64 tokens at decode batch 64, so only
+// 64 workgroups): the row's loads are spread over as many threads as there
+// are; 256 took 10.9 us for the qkv row of Llama-3-8B at batch 64, more than
+// the separate reduce and rotary kernels together.
 constexpr int kThreads = 1024;
 
 struct KParams {
@@ -268,7 +268,7 @@ template <typename E>
 __device__ __forceinline__ void reduce_row(const KParams& p, int t) {
   const float* prow = p.part + static_cast<int64_t>(t) * p.N;
   uint16_t* crow = p.C + static_cast<int64_t>(t) * p.ldc;
-  for (int n = 4 * static_cast<int>(threadIdx.x); n < p.N; n += 4 * kThreads) {
+  for (int n = 4 * static_cast<int>(threadIdx.x); n < p.N; n += 4 * static_cast<int>(blockDim.x)) {
     float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     if (p.N % 4 == 0) {
       // Every split's 16 bytes are loaded before the in-order sum, so one
@@ -341,7 +341,7 @@ __global__ __launch_bounds__(kThreads) void rotary_and_cache_kernel(const KParam
   using CE = std::conditional_t<FP8, uint8_t, uint16_t>;
   CE* const kcb = reinterpret_cast<CE*>(c.kc) + blk * c.kc_sb + off * c.kc_st;
   CE* const vcb = reinterpret_cast<CE*>(c.vc) + blk * c.vc_sb + off * c.vc_st;
-  for (int it = threadIdx.x; it < rot_items + copy_items; it += kThreads) {
+  for (int it = threadIdx.x; it < rot_items + copy_items; it += static_cast<int>(blockDim.x)) {
     if (it < rot_items) {
       const int h = it / steps;
       const int i0 = (it - h * steps) * VW;
@@ -460,9 +460,26 @@ __global__ __launch_bounds__(kThreads) void rotary_and_cache_kernel(const KParam
   }
 }
 
+// Threads of a token's workgroup. The scalar path (four to eight times the
+// items) and the split-K input take kThreads. Otherwise no wave without an
+// item, and at most 512 threads below 768 tokens (3 workgroups a CU), 256 from
+// there on: with few workgroups a token's items are a chain that more threads
+// shorten, with many the chip is full and a wave of one item pays its start for
+// 16 bytes. us at 1024 / 512 / 256 threads, heads + KV heads x head_dim, bf16:
+//   32 + 8 x 128: 64 tokens 3.58 / 3.45 / 3.88, 512 tokens 5.80 / 5.28 / 5.42,
+//     1003 tokens 9.48 / 7.79 / 7.77, 4096 tokens 27.4 / 20.5 / 18.7 (the last
+//     6 TB/s of the 112 MB that are read and written);
+//   28 + 4 x 128: 1003 tokens 8.48 / 6.96 / 6.76, 4096 tokens 25.4 / 17.7 / 15.4;
+//   14 + 2 x 64 (144 items, so 192 threads): 4096 tokens 18.6, with 192 8.5.
+inline int threads(const KParams& p, bool vec) {
+  if (!vec || p.part != nullptr) return kThreads;
+  const int items = (p.r.hq + p.r.hkv) * (p.r.rot_dim / 8) + p.c.hkv * ((2 * p.c.d - p.r.rot_dim) / 8);
+  return min(p.r.num_tokens < 768 ? 512 : 256, (items + 63) / 64 * 64);
+}
+
 template <typename E, typename CT, bool FP8>
 hipError_t launch(const KParams& kp, bool neox, bool vec, float k_scale, float v_scale, hipStream_t s) {
-  const dim3 grid(kp.r.num_tokens), block(kThreads);
+  const dim3 grid(kp.r.num_tokens), block(threads(kp, vec));
   if (neox) {
     if (vec) hipLaunchKernelGGL((rotary_and_cache_kernel<E, CT, true, true, FP8>), grid, block, 0, s, kp, k_scale, v_scale);
     else hipLaunchKernelGGL((rotary_and_cache_kernel<E, CT, true, false, FP8>), grid, block, 0, s, kp, k_scale, v_scale);

@@ -315,6 +315,27 @@ def test_fused_rope_and_cache_equals_the_two_ops(dtype, is_neox, head_size, rot_
     assert torch.equal(kv.k_cache.cpu(), want_kc) and torch.equal(kv.v_cache.cpu(), want_vc)
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("is_neox", [True, False])
+@pytest.mark.parametrize("tokens", [1, 767, 768])
+@pytest.mark.parametrize("hq,hkv,d,rot_dim", [(32, 8, 128, 128), (28, 4, 128, 64), (14, 2, 64, 64), (1, 1, 64, 64)])
+def test_fused_rope_and_cache_workgroup_sizes(fp8, is_neox, tokens, hq, hkv, d, rot_dim):
+    """Vector path, with 768, 352, 144 and 24 items a token: several passes of
+    512 (below 768 tokens) or 256 threads, a part-filled last wave, one wave.
+    Bit for bit the two ops in sequence."""
+    dtype = torch.bfloat16
+    kv = make_paged_kv([900, 300], hkv, d, 16, FP8 if fp8 else dtype, "cuda", layout="nhd", seed=tokens)
+    g = torch.Generator(device="cuda").manual_seed(tokens + hq)
+    buf = torch.randn(tokens, (hq + 2 * hkv) * d, generator=g, device="cuda", dtype=dtype)
+    q, k, v = buf.split([hq * d, hkv * d, hkv * d], dim=1)
+    cache = rope_cos_sin_cache(4096, rot_dim).cuda()
+    slots = _slots(kv.k_cache.shape[0], 16, tokens, seed=hq)
+    scales = dict(k_scale=0.5, v_scale=2.0) if fp8 else {}
+    fused, pair = _run_fused_and_pair(kv, buf, q, k, v, cache, _positions(tokens, 4096, 7), slots, d, is_neox, **scales)
+    for name, a, b in zip(("query", "key", "key_cache", "value_cache"), fused, pair):
+        assert torch.equal(a, b), f"fused {name} differs from rotary_embedding + reshape_and_cache"
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("is_neox", [True, False])
 @pytest.mark.parametrize("case", ["misaligned_rows", "rot_dim_36"])
