@@ -376,7 +376,7 @@ __device__ __forceinline__ void dma_tile_of(int id, int tiles_m, int tiles_n, in
 struct KWalk {
   int kb, end, ktiles, rot;
   __device__ __forceinline__ KWalk(int kb_, int ktiles_, int rot_)
-      : kb(kb_), end(kb_ + ktiles_ * kDmaBK), ktiles(ktiles_), rot(ktiles_ > 0 ? rot_ % ktiles_ : 0) {}
+      : kb(kb_), end(kb_ + ktiles_ * kDmaBK), ktiles(ktiles_), rot(rot_ > 0 && ktiles_ > 0 ? rot_ % ktiles_ : 0) {}
   // First column of the walk's slice t; past the range for t >= ktiles.
   __device__ __forceinline__ int at(int t) const {
     const int r = t + rot;
@@ -563,20 +563,24 @@ __device__ __forceinline__ void ring_tile(const uint16_t* __restrict__ A, const 
   const int ktiles = (ke - kb + kDmaBK - 1) / kDmaBK;
   const int full = (ke - kb) / kDmaBK;  // slices that lie wholly inside the K range
   const KWalk walk(kb, ktiles, full == ktiles ? tn * rot_step : 0);
-  // Slice t of the walk into ring buffer `buf`. Checked: also for slices that
+  // The slice at column k0 into ring buffer `buf`. Checked: also for slices that
   // end past the K range, or start there (those lanes are out of range and move
   // no data), so that each wave keeps the same count in flight from slice to
-  // slice. Whole slices take their K offset as the load's scalar offset, which
-  // leaves no vector arithmetic in the steady loop, and `k0` steps with the
-  // walk (a compare and a select per slice).
+  // slice. Whole slices need one addition per load (rows past M or N stay out
+  // of range: kNowhere + 2 k0 is still above every resource's extent), and `k0`
+  // steps with the walk (a compare and a select per slice). With the K offset
+  // as the loads' scalar offset instead, as in the ping-pong body, the larger
+  // tiles were 1-6% slower (us): 128 x 128 at M, N, K = 192, 16384, 3072 36.4
+  // against 34.3 and at 768, 3584, 3584 36.5 against 34.9, 192 x 224 at 768,
+  // 28672, 4096 177 against 168.
   auto issue = [&](bool checked, int k0, int buf) {
     u32x4* base = lds + buf * kSlice;
     const bool in = k0 + kc < ke;
 #pragma unroll
     for (int j = 0; j < LA; ++j) {
-      const int off = static_cast<int>(checked ? (in ? offa[j] + 2 * k0 : kNowhere) : offa[j]);
+      const int off = static_cast<int>(!checked || in ? offa[j] + 2 * k0 : kNowhere);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          ra, (__attribute__((address_space(3))) void*)(base + (wave + j * NW) * 64), 16, off, checked ? 0 : 2 * k0, 0, 0);
+          ra, (__attribute__((address_space(3))) void*)(base + (wave + j * NW) * 64), 16, off, 0, 0, 0);
     }
 #pragma unroll
     for (int j = 0; j < LB; ++j) {
@@ -585,9 +589,9 @@ __device__ __forceinline__ void ring_tile(const uint16_t* __restrict__ A, const 
         if (!kSpare) break;
         to = lds + STAGES * kSlice;
       }
-      const int off = static_cast<int>(checked ? (in ? offb[j] + 2 * k0 : kNowhere) : offb[j]);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (__attribute__((address_space(3))) void*)to, 16, off,
-                                               checked ? 0 : 2 * k0, 0, 0);
+      const int off = static_cast<int>(!checked || in ? offb[j] + 2 * k0 : kNowhere);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (__attribute__((address_space(3))) void*)to, 16, off, 0,
+                                               0, 0);
     }
   };
 
