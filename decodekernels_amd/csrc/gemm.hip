@@ -30,6 +30,7 @@
 //   where they fill the CUs, for N > 32768 (decode_dma_plan), and where they
 //   measured faster at any M (decode_tile_plan).
 #include <algorithm>
+#include <type_traits>
 
 #include "../../include/decodekernels_amd.h"
 #include "dk_device.h"
@@ -467,6 +468,37 @@ __device__ __forceinline__ void store_tile(const f32x4 (&acc)[TM][TN], u32x4* ld
     }
   }
   __syncthreads();  // the tile's rows come from the other lanes of the wave
+  if (vec_store <= 0) {
+    // Rows that allow only 4- or 2-byte stores: consecutive lanes take
+    // consecutive columns, so that a store still writes whole row segments. (As
+    // pieces of each lane's own 16 bytes, a store touched 64 pieces of 4 to 8
+    // rows, up to 40% of a call: M, N, K = 1108, 11013, 368 40.0 -> 24.9 us, 3976,
+    // 22398, 336 228 -> 132, in 256 x 256 tiles; 128 x 128 tiles 1.2 times faster
+    // on average, 64 x 64 1.05. In a grid of 2 x 4 waves a row's segment is half
+    // as long as in 4 x 2, which had cost another 5%.)
+    const auto narrow = [&](auto width) {
+      constexpr int kW = decltype(width)::value;  // columns per store
+      constexpr int kPerRow = 16 * TN / kW;
+#pragma unroll 4
+      for (int it = 0; it < 16 * TM * kPerRow / kWave; ++it) {
+        const int idx = it * kWave + lane;
+        const int row = idx / kPerRow;
+        const int c = idx % kPerRow * kW;
+        const char* from = stg + row * kPitch + 2 * c;
+        const int m = m0 + row;
+        const int n = n0 + c;
+        if (m >= M || n >= N) continue;
+        uint16_t* to = C + static_cast<int64_t>(m) * ldc + n;
+        if (kW == 2 && n + 1 < N)
+          *reinterpret_cast<uint32_t*>(to) = *reinterpret_cast<const uint32_t*>(from);
+        else
+          *to = *reinterpret_cast<const uint16_t*>(from);
+      }
+    };
+    if (vec_store == 0) narrow(std::integral_constant<int, 2>{});
+    else narrow(std::integral_constant<int, 1>{});
+    return;
+  }
   constexpr int kChunks = 16 * TM * kNc;  // 16-byte chunks of a wave's tile
 #pragma unroll
   for (int it = 0; it < (kChunks + kWave - 1) / kWave; ++it) {
@@ -479,11 +511,13 @@ __device__ __forceinline__ void store_tile(const f32x4 (&acc)[TM][TN], u32x4* ld
     const int n = n0 + 8 * c;
     if (m >= M) continue;
     uint16_t* crow = C + static_cast<int64_t>(m) * ldc;
-    if (vec_store == 2 && n + 7 < N) {
-      *reinterpret_cast<u32x4*>(crow + n) = val;
-    } else if (vec_store == 1 && n + 7 < N) {
-      *reinterpret_cast<u32x2*>(crow + n) = u32x2{val[0], val[1]};
-      *reinterpret_cast<u32x2*>(crow + n + 4) = u32x2{val[2], val[3]};
+    if (n + 7 < N) {
+      if (vec_store == 2) {
+        *reinterpret_cast<u32x4*>(crow + n) = val;
+      } else {
+        *reinterpret_cast<u32x2*>(crow + n) = u32x2{val[0], val[1]};
+        *reinterpret_cast<u32x2*>(crow + n + 4) = u32x2{val[2], val[3]};
+      }
     } else {
 #pragma unroll
       for (int r = 0; r < 8; ++r)
@@ -714,12 +748,10 @@ __device__ __forceinline__ void ring_tile(const uint16_t* __restrict__ A, const 
 // loads' scalar offset (with it in the vector offset, and compared with the K
 // range per lane, the 256 x 256 tile took 674 us on gate_up at M = 4096, with
 // the ring body 741; now 643, hipBLASLt 641, same run). M = N = 4096: K = 4096
-// 112.5 -> 93.2 us, K = 14336 383 -> 346 us. Loads alone take 256 us of the
-// latter, MFMAs alone 227 us. Waiting for the reads only when they are used,
-// without the raised priority, with the loads in two phases instead of four,
-// or starting each XCD at another K offset were all within 1%.
-//
-// A square tile's waves form a 2 x 4 grid (1-2% faster than 4 x 2).
+// 112.5 -> 93.2 us, K = 14336 383 -> 346 us. Waiting for the reads only when
+// they are used, without the raised priority, with the loads in two phases
+// instead of four, or starting each XCD at another K offset were all within 1%.
+
 // A barrier that neither LDS reads nor loads into LDS are moved across.
 __device__ __forceinline__ void pp_barrier() {
   __builtin_amdgcn_sched_barrier(0);
@@ -739,13 +771,11 @@ __device__ __forceinline__ void pp_wait_barrier() {
   pp_barrier();
 }
 
-template <typename E, int BM, int BN, int GM, int GN>
+template <typename E, int BM, int BN, int WM, int WN>
 __device__ __forceinline__ void ping_pong_tile(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
                                                const uint16_t* __restrict__ bias, uint16_t* __restrict__ C, int M,
                                                int N, int K, int lda, int ldb, int ldc, int vec_store,
                                                float* __restrict__ part, int k_split, int rot_step) {
-  constexpr int WM = BM == BN ? GN : GM;
-  constexpr int WN = BM == BN ? GM : GN;
   constexpr int NW = WM * WN;
   static_assert(NW == 8, "two waves per SIMD, one of each half of the workgroup");
   constexpr int QR = BM / 2 / WM;  // rows of A (of B) of one half that a wave multiplies
@@ -963,8 +993,11 @@ template <typename E, int BM, int BN, int WM, int WN, int STAGES>
 hipError_t launch_dma(const uint16_t* A, const uint16_t* B, const uint16_t* bias, uint16_t* C, int M, int N, int K,
                       int lda, int ldb, int ldc, hipStream_t s, float* part, int splits, int k_split, bool reduce, int rot_step) {
   const int64_t tiles = ceil_div64(M, BM) * ceil_div64(N, BN);
-  // Output stores of 16 bytes, or 8 where C's rows allow only that.
-  const int vec = (ldc % 8 == 0 && aligned_to(C, 16)) ? 2 : (ldc % 4 == 0 && aligned_to(C, 8)) ? 1 : 0;
+  // Output stores of 16 bytes (2), or 8 (1), 4 (0) or 2 (-1) where C's rows allow only that.
+  const int vec = (ldc % 8 == 0 && aligned_to(C, 16))  ? 2
+                  : (ldc % 4 == 0 && aligned_to(C, 8)) ? 1
+                  : (ldc % 2 == 0 && aligned_to(C, 4)) ? 0
+                                                       : -1;
   hipLaunchKernelGGL((gemm_dma_kernel<E, BM, BN, WM, WN, STAGES>),
                      dim3(static_cast<unsigned>(tiles), static_cast<unsigned>(part != nullptr ? splits : 1)),
                      dim3(WM * WN * kWave), 0, s, A, B, bias, C, M, N, K, lda, ldb, ldc, vec, part,
@@ -979,11 +1012,12 @@ hipError_t launch_dma(const uint16_t* A, const uint16_t* B, const uint16_t* bias
 using DmaLauncher = hipError_t (*)(const uint16_t*, const uint16_t*, const uint16_t*, uint16_t*, int, int, int, int,
                                    int, int, hipStream_t, float*, int, int, bool, int);
 
-// Launchers of kTileShapes' tile shapes, in the same order.
+// Launchers of kTileShapes' tile shapes, in the same order. The waves of the
+// 256 x 256 tile form a 2 x 4 grid (0-2% faster than 4 x 2).
 template <typename E>
 const DmaLauncher* tile_launchers() {
   static const DmaLauncher fns[] = {
-      launch_dma<E, 256, 256, 4, 2, 2>, launch_dma<E, 256, 192, 4, 2, 2>, launch_dma<E, 192, 256, 2, 4, 2>,
+      launch_dma<E, 256, 256, 2, 4, 2>, launch_dma<E, 256, 192, 4, 2, 2>, launch_dma<E, 192, 256, 2, 4, 2>,
       launch_dma<E, 256, 128, 4, 2, 2>, launch_dma<E, 128, 256, 2, 4, 2>, launch_dma<E, 128, 128, 4, 2, 3>,
       launch_dma<E, 128, 160, 4, 2, 4>, launch_dma<E, 128, 64, 2, 2, 4>,  launch_dma<E, 64, 64, 2, 2, 4>,
       launch_dma<E, 64, 128, 2, 2, 4>,  launch_dma<E, 192, 192, 4, 2, 3>, launch_dma<E, 192, 224, 4, 2, 2>,

@@ -212,3 +212,27 @@ def test_tile_against_fp32(tile, bf16):
             assert rc == 0, capi.last_error()
             torch.cuda.synchronize()
             assert torch.equal(c, d)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", [(64, 64, False, 0), (128, 160, False, 0), (256, 128, False, 0), (256, 256, False, 0)])
+def test_output_rows_of_any_alignment(tile):
+    """Stores of 16, 8, 4 and 2 bytes: output rows of every stride modulo 8
+    starting at every element offset modulo 8, odd and even N; the elements
+    around each row keep their values."""
+    from parity import assert_max_abs, gemm_f32_gpu
+
+    M, N, K = SHAPES[tile][0]
+    for n in (N, N - 1, N - 2):
+        g = torch.Generator(device="cuda").manual_seed(n)
+        a = torch.randn(M, K, generator=g, device="cuda", dtype=torch.bfloat16)
+        b = torch.randn(n, K, generator=g, device="cuda", dtype=torch.bfloat16) / K**0.5
+        bias = torch.randn(n, generator=g, device="cuda", dtype=torch.bfloat16)
+        want = gemm_f32_gpu(a, b, bias)
+        for pad, at in [(0, 0), (0, 1), (1, 0), (2, 2), (3, 3), (4, 4), (5, 1), (6, 2), (7, 5), (8, 6), (8, 8)]:
+            print(f"gemm {M}x{n}x{K} tile {capi.gemm_tile(M, n, K)} row stride {n + pad}, first element {at}", flush=True)
+            flat = torch.full((at + M * (n + pad) + 8,), float("nan"), device="cuda", dtype=torch.bfloat16)
+            out = flat[at : at + M * (n + pad)].view(M, n + pad)[:, :n]
+            torch.ops.decode_kernels.gemm_tn(out, a, b, bias)
+            assert_max_abs(out, want, torch.bfloat16, f"gemm {M}x{n}x{K}, row stride {n + pad}, first element {at}")
+            assert int(flat.isnan().sum()) == at + M * pad + 8

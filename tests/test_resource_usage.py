@@ -93,7 +93,7 @@ OCCUPANCY = [
     (("paged_attention_balanced_kernel<dk::Bf16, 64, true, 16, 4, false>",), 4),
     (("paged_attention_balanced_kernel<dk::Bf16, 256, true, 16, 2, false>",), 1),
     (("paged_attention_reduce_kernel<dk::Bf16, 128",), 8),
-    (("gemm_dma_kernel<dk::Bf16, 256, 256, 4, 2, 2>",), 2),
+    (("gemm_dma_kernel<dk::Bf16, 256, 256, 2, 4, 2>",), 2),
     (("gemm_dma_kernel<dk::Bf16, 256, 192, 4, 2, 2>",), 2),
     (("gemm_dma_kernel<dk::Bf16, 256, 224, 4, 2, 2>",), 2),
     (("gemm_dma_kernel<dk::Bf16, 192, 192, 4, 2, 3>",), 2),
