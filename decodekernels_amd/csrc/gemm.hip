@@ -468,14 +468,15 @@ __device__ __forceinline__ void store_tile(const f32x4 (&acc)[TM][TN], u32x4* ld
     }
   }
   __syncthreads();  // the tile's rows come from the other lanes of the wave
-  if (vec_store <= 0) {
-    // Rows that allow only 4- or 2-byte stores: consecutive lanes take
-    // consecutive columns, so that a store still writes whole row segments. (As
-    // pieces of each lane's own 16 bytes, a store touched 64 pieces of 4 to 8
-    // rows, up to 40% of a call: M, N, K = 1108, 11013, 368 40.0 -> 24.9 us, 3976,
-    // 22398, 336 228 -> 132, in 256 x 256 tiles; 128 x 128 tiles 1.2 times faster
-    // on average, 64 x 64 1.05. In a grid of 2 x 4 waves a row's segment is half
-    // as long as in 4 x 2, which had cost another 5%.)
+  if (vec_store <= 0 || (N % 8 != 0 && n0 + 16 * TN > N)) {
+    // Rows that allow only 4- or 2-byte stores, and the last columns of an N that
+    // is no multiple of a lane's 8: consecutive lanes take consecutive columns, so
+    // that a store still writes whole row segments. (As pieces of each lane's own
+    // 16 bytes, a store touched 64 pieces of 4 to 8 rows, up to 40% of a call: M,
+    // N, K = 1108, 11013, 368 40.0 -> 24.9 us, 3976, 22398, 336 228 -> 132, in 256
+    // x 256 tiles; 128 x 128 tiles 1.2 times faster on average, 64 x 64 1.05. In a
+    // grid of 2 x 4 waves a row's segment is half as long as in 4 x 2, which had
+    // cost another 5%.)
     const auto narrow = [&](auto width) {
       constexpr int kW = decltype(width)::value;  // columns per store
       constexpr int kPerRow = 16 * TN / kW;
@@ -495,7 +496,7 @@ __device__ __forceinline__ void store_tile(const f32x4 (&acc)[TM][TN], u32x4* ld
           *to = *reinterpret_cast<const uint16_t*>(from);
       }
     };
-    if (vec_store == 0) narrow(std::integral_constant<int, 2>{});
+    if (vec_store >= 0) narrow(std::integral_constant<int, 2>{});
     else narrow(std::integral_constant<int, 1>{});
     return;
   }
@@ -509,19 +510,13 @@ __device__ __forceinline__ void store_tile(const f32x4 (&acc)[TM][TN], u32x4* ld
     const u32x4 val = *reinterpret_cast<const u32x4*>(stg + row * kPitch + c * 16);
     const int m = m0 + row;
     const int n = n0 + 8 * c;
-    if (m >= M) continue;
-    uint16_t* crow = C + static_cast<int64_t>(m) * ldc;
-    if (n + 7 < N) {
-      if (vec_store == 2) {
-        *reinterpret_cast<u32x4*>(crow + n) = val;
-      } else {
-        *reinterpret_cast<u32x2*>(crow + n) = u32x2{val[0], val[1]};
-        *reinterpret_cast<u32x2*>(crow + n + 4) = u32x2{val[2], val[3]};
-      }
+    if (m >= M || n >= N) continue;
+    uint16_t* to = C + static_cast<int64_t>(m) * ldc + n;
+    if (vec_store == 2) {
+      *reinterpret_cast<u32x4*>(to) = val;
     } else {
-#pragma unroll
-      for (int r = 0; r < 8; ++r)
-        if (n + r < N) crow[n + r] = static_cast<uint16_t>(val[r / 2] >> (16 * (r % 2)));
+      *reinterpret_cast<u32x2*>(to) = u32x2{val[0], val[1]};
+      *reinterpret_cast<u32x2*>(to + 4) = u32x2{val[2], val[3]};
     }
   }
 }
