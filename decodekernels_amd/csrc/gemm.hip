@@ -376,8 +376,14 @@ __device__ __forceinline__ void dma_tile_of(int id, int tiles_m, int tiles_n, in
 // from slice `rot` on, round to slice rot - 1 (rot = 0: in order).
 struct KWalk {
   int kb, end, ktiles, rot;
-  __device__ __forceinline__ KWalk(int kb_, int ktiles_, int rot_)
-      : kb(kb_), end(kb_ + ktiles_ * kDmaBK), ktiles(ktiles_), rot(rot_ > 0 && ktiles_ > 0 ? rot_ % ktiles_ : 0) {}
+  // rot_inv: 0, or 2^32 / ktiles rounded up, for column tile tn to start at slice
+  // tn mod ktiles (exact for tn ktiles < 2^32; an integer division in every
+  // workgroup showed in the shortest calls).
+  __device__ __forceinline__ KWalk(int kb_, int ktiles_, int tn, unsigned rot_inv)
+      : kb(kb_),
+        end(kb_ + ktiles_ * kDmaBK),
+        ktiles(ktiles_),
+        rot(rot_inv != 0 ? max(0, tn - static_cast<int>(__umulhi(tn, rot_inv)) * ktiles_) : 0) {}
   // First column of the walk's slice t; past the range for t >= ktiles.
   __device__ __forceinline__ int at(int t) const {
     const int r = t + rot;
@@ -527,7 +533,7 @@ template <typename E, int BM, int BN, int WM, int WN, int STAGES>
 __device__ __forceinline__ void ring_tile(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
                                           const uint16_t* __restrict__ bias, uint16_t* __restrict__ C, int M, int N,
                                           int K, int lda, int ldb, int ldc, int vec_store, float* __restrict__ part,
-                                          int k_split, int rot_step) {
+                                          int k_split, unsigned rot_inv) {
   constexpr int NW = WM * WN;
   constexpr int TM = BM / WM / 16;  // 16-row fragments per wave
   constexpr int TN = BN / WN / 16;
@@ -591,7 +597,7 @@ __device__ __forceinline__ void ring_tile(const uint16_t* __restrict__ A, const 
   }
   const int ktiles = (ke - kb + kDmaBK - 1) / kDmaBK;
   const int full = (ke - kb) / kDmaBK;  // slices that lie wholly inside the K range
-  const KWalk walk(kb, ktiles, full == ktiles ? tn * rot_step : 0);
+  const KWalk walk(kb, ktiles, tn, rot_inv);
   // The slice at column k0 into ring buffer `buf`. Checked: also for slices that
   // end past the K range, or start there (those lanes are out of range and move
   // no data), so that each wave keeps the same count in flight from slice to
@@ -604,10 +610,10 @@ __device__ __forceinline__ void ring_tile(const uint16_t* __restrict__ A, const 
   // 28672, 4096 177 against 168.
   auto issue = [&](bool checked, int k0, int buf) {
     u32x4* base = lds + buf * kSlice;
-    const bool in = k0 + kc < ke;
+    const unsigned out = checked && k0 + kc >= ke ? kNowhere : 0;  // or-ed in: a choice per load became a branch
 #pragma unroll
     for (int j = 0; j < LA; ++j) {
-      const int off = static_cast<int>(!checked || in ? offa[j] + 2 * k0 : kNowhere);
+      const int off = static_cast<int>((offa[j] + 2 * k0) | out);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           ra, (__attribute__((address_space(3))) void*)(base + (wave + j * NW) * 64), 16, off, 0, 0, 0);
     }
@@ -618,7 +624,7 @@ __device__ __forceinline__ void ring_tile(const uint16_t* __restrict__ A, const 
         if (!kSpare) break;
         to = lds + STAGES * kSlice;
       }
-      const int off = static_cast<int>(!checked || in ? offb[j] + 2 * k0 : kNowhere);
+      const int off = static_cast<int>((offb[j] + 2 * k0) | out);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (__attribute__((address_space(3))) void*)to, 16, off, 0,
                                                0, 0);
     }
@@ -770,7 +776,7 @@ template <typename E, int BM, int BN, int WM, int WN>
 __device__ __forceinline__ void ping_pong_tile(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
                                                const uint16_t* __restrict__ bias, uint16_t* __restrict__ C, int M,
                                                int N, int K, int lda, int ldb, int ldc, int vec_store,
-                                               float* __restrict__ part, int k_split, int rot_step) {
+                                               float* __restrict__ part, int k_split, unsigned rot_inv) {
   constexpr int NW = WM * WN;
   static_assert(NW == 8, "two waves per SIMD, one of each half of the workgroup");
   constexpr int QR = BM / 2 / WM;  // rows of A (of B) of one half that a wave multiplies
@@ -833,15 +839,15 @@ __device__ __forceinline__ void ping_pong_tile(const uint16_t* __restrict__ A, c
   }
   const int ktiles = (ke - kb + kDmaBK - 1) / kDmaBK;
   const int full = (ke - kb) / kDmaBK;
-  const KWalk walk(kb, ktiles, full == ktiles ? tn * rot_step : 0);
+  const KWalk walk(kb, ktiles, tn, rot_inv);
   // The loads of half `i` of the slice at column k0 into buffer `buf`. Checked:
   // also for slices that end past the K range (or start there: nothing is moved).
   auto issue_a = [&](bool checked, int k0, int buf, int i) {
     u32x4* base = lds + buf * kSlice + i * kHalfA;
-    const bool in = k0 + kc < ke;
+    const unsigned out = k0 + kc < ke ? 0 : kNowhere;
 #pragma unroll
     for (int j = 0; j < LA; ++j) {
-      const int off = static_cast<int>(checked ? (in ? offa[i][j] + 2 * k0 : kNowhere) : offa[i][j]);
+      const int off = static_cast<int>(checked ? (offa[i][j] + 2 * k0) | out : offa[i][j]);
       u32x4* to = wave + j * NW < kGroupsA ? base + (wave + j * NW) * 64 : lds + 2 * kSlice;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (__attribute__((address_space(3))) void*)to, 16, off,
                                                checked ? 0 : 2 * k0, 0, 0);
@@ -849,10 +855,10 @@ __device__ __forceinline__ void ping_pong_tile(const uint16_t* __restrict__ A, c
   };
   auto issue_b = [&](bool checked, int k0, int buf, int i) {
     u32x4* base = lds + buf * kSlice + 2 * kHalfA + i * kHalfB;
-    const bool in = k0 + kc < ke;
+    const unsigned out = k0 + kc < ke ? 0 : kNowhere;
 #pragma unroll
     for (int j = 0; j < LB; ++j) {
-      const int off = static_cast<int>(checked ? (in ? offb[i][j] + 2 * k0 : kNowhere) : offb[i][j]);
+      const int off = static_cast<int>(checked ? (offb[i][j] + 2 * k0) | out : offb[i][j]);
       u32x4* to = wave + j * NW < kGroupsB ? base + (wave + j * NW) * 64 : lds + 2 * kSlice;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (__attribute__((address_space(3))) void*)to, 16, off,
                                                checked ? 0 : 2 * k0, 0, 0);
@@ -974,11 +980,11 @@ __global__ __launch_bounds__(WM * WN * kWave, 2) void gemm_dma_kernel(const uint
                                                                    const uint16_t* __restrict__ bias,
                                                                    uint16_t* __restrict__ C, int M, int N, int K,
                                                                    int lda, int ldb, int ldc, int vec_store,
-                                                                   float* __restrict__ part, int k_split, int rot_step) {
+                                                                   float* __restrict__ part, int k_split, unsigned rot_inv) {
   if constexpr (ping_pong<BN, STAGES>())
-    ping_pong_tile<E, BM, BN, WM, WN>(A, B, bias, C, M, N, K, lda, ldb, ldc, vec_store, part, k_split, rot_step);
+    ping_pong_tile<E, BM, BN, WM, WN>(A, B, bias, C, M, N, K, lda, ldb, ldc, vec_store, part, k_split, rot_inv);
   else
-    ring_tile<E, BM, BN, WM, WN, STAGES>(A, B, bias, C, M, N, K, lda, ldb, ldc, vec_store, part, k_split, rot_step);
+    ring_tile<E, BM, BN, WM, WN, STAGES>(A, B, bias, C, M, N, K, lda, ldb, ldc, vec_store, part, k_split, rot_inv);
 }
 #pragma clang diagnostic pop
 
@@ -988,6 +994,7 @@ template <typename E, int BM, int BN, int WM, int WN, int STAGES>
 hipError_t launch_dma(const uint16_t* A, const uint16_t* B, const uint16_t* bias, uint16_t* C, int M, int N, int K,
                       int lda, int ldb, int ldc, hipStream_t s, float* part, int splits, int k_split, bool reduce, int rot_step) {
   const int64_t tiles = ceil_div64(M, BM) * ceil_div64(N, BN);
+  const unsigned rot_inv = rot_step != 0 ? static_cast<unsigned>(ceil_div64(int64_t{1} << 32, K / kDmaBK)) : 0;
   // Output stores of 16 bytes (2), or 8 (1), 4 (0) or 2 (-1) where C's rows allow only that.
   const int vec = (ldc % 8 == 0 && aligned_to(C, 16))  ? 2
                   : (ldc % 4 == 0 && aligned_to(C, 8)) ? 1
@@ -996,7 +1003,7 @@ hipError_t launch_dma(const uint16_t* A, const uint16_t* B, const uint16_t* bias
   hipLaunchKernelGGL((gemm_dma_kernel<E, BM, BN, WM, WN, STAGES>),
                      dim3(static_cast<unsigned>(tiles), static_cast<unsigned>(part != nullptr ? splits : 1)),
                      dim3(WM * WN * kWave), 0, s, A, B, bias, C, M, N, K, lda, ldb, ldc, vec, part,
-                     part != nullptr ? k_split : K, rot_step);
+                     part != nullptr ? k_split : K, rot_inv);
   if (part == nullptr || !reduce) return hipGetLastError();
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
@@ -1302,12 +1309,14 @@ constexpr TileShape kDecodeShapes[] = {{64, 64, 0.207, 0.519, true}, {64, 128, 0
 // K-walk rotation (see gemm_skinny_lds_kernel): column tile j starts its walk
 // j slices in. With one tile row every weight byte is read by one workgroup,
 // and spreading the walks spreads the reads over the HBM channels where rows
-// are 8 KB or 16 KB apart: gate_up (N 28672, K 4096) at M = 64 / 128 / 250
-// 52.4 / 57.8 / 69.5 -> 42.2 / 50.0 / 62.5 us, N = 128256 at M = 16 219 -> 176;
-// at K = 3584 and 5120 within 1%. With more tile rows, whose workgroups share
-// weight rows, and below 128 workgroups it measured 0-4% slower.
-inline int rotation(int64_t tiles_m, int64_t tiles_n, int splits) {
-  return splits == 1 && tiles_m == 1 && tiles_n >= 128 ? 1 : 0;
+// are a few KB apart: gate_up (N 28672, K 4096) at M = 64 / 128 / 250 52.4 / 57.8 /
+// 69.5 -> 42.2 / 50.0 / 62.5 us, N = 128256 at M = 16 219 -> 176. By K, over ten
+// tiles and eight widths: 0.91-0.93 of the time in order at 2048, 4096, 6144,
+// 8192 and 16384, 0.97-0.99 at 1536, 2560, 3072, 3584, 9216, 1.00 up to 1024
+// (N 9728, K 1024 at M = 65 9.4 -> 10.0). With more tile rows, whose workgroups
+// share weight rows, and below 128 workgroups it measured 0-4% slower.
+inline int rotation(int64_t tiles_m, int64_t tiles_n, int splits, int K) {
+  return splits == 1 && tiles_m == 1 && tiles_n >= 128 && K >= 1536 && K % kDmaBK == 0 ? 1 : 0;
 }
 
 inline TilePlan fastest_tile(const TileModel& m, const TileShape* shapes, int count, int M, int N, int K,
@@ -1342,7 +1351,7 @@ inline TilePlan fastest_tile(const TileModel& m, const TileShape* shapes, int co
       if (s > 1) t += m.split + m.per_split * s + s * mn * 8.0 / m.partials;
       t = t * t * t * t + mem4;
       if (best_t < 0 || t < best_t) {
-        best = TilePlan{i, s, ks, rotation(tiles_m, tiles_n, s)};
+        best = TilePlan{i, s, ks, rotation(tiles_m, tiles_n, s, K)};
         best_t = t;
       }
     }
@@ -1442,10 +1451,10 @@ inline int64_t decode_dma_workspace_bytes(const DecodeDmaPlan& d, int M, int N) 
 inline TilePlan decode_tile_plan(int M, int N, int K, int plan_splits) {
   const int64_t t128 = ceil_div64(N, 128);
   const int64_t t64 = ceil_div64(N, 64);
-  if (K >= 2048 && t64 >= 192 && t64 <= kSkinnyCus) return TilePlan{kTile64x64, 1, K, rotation(1, t64, 1)};
+  if (K >= 2048 && t64 >= 192 && t64 <= kSkinnyCus) return TilePlan{kTile64x64, 1, K, rotation(1, t64, 1, K)};
   if (K >= 2048 && plan_splits == 1 && t64 > kSkinnyCus &&
       4 * t128 >= 3 * kSkinnyCus * ceil_div64(t128, kSkinnyCus))
-    return TilePlan{kTile64x128, 1, K, rotation(1, t128, 1)};
+    return TilePlan{kTile64x128, 1, K, rotation(1, t128, 1, K)};
   if (plan_splits < 3) return TilePlan{-1, 1, K, 0};
   TilePlan t = fastest_tile(kDecodeModel, kDecodeShapes, 2, M, N, K, plan_splits);
   t.shape = t.shape == 0 ? kTile64x64 : kTile64x128;
@@ -1532,7 +1541,7 @@ hipError_t launch(const uint16_t* A, const uint16_t* B, const uint16_t* bias, ui
       if (deferred_splits != nullptr) *deferred_splits = d.splits;
       return tile_launchers<E>()[d.bn == 64 ? kTile64x64 : kTile64x128](
           A, B, bias, C, M, N, K, lda, ldb, ldc, s, d.splits > 1 ? static_cast<float*>(workspace) : nullptr, d.splits,
-          d.k_split, deferred_splits == nullptr, rotation(1, ceil_div64(N, d.bn), d.splits));
+          d.k_split, deferred_splits == nullptr, rotation(1, ceil_div64(N, d.bn), d.splits, K));
     }
     float* part = p.splits > 1 ? static_cast<float*>(workspace) : nullptr;
     if (deferred_splits != nullptr) *deferred_splits = p.splits;
@@ -1674,7 +1683,7 @@ extern "C" int dk_gemm_tn_tile(int M, int N, int K, int with_workspace, int* til
     tile[0] = plan[0];
     tile[1] = plan[1];
     tile[2] = plan[2];
-    tile[3] = plan[0] == 64 ? rotation(1, ceil_div64(N, plan[1]), plan[2]) : 0;
+    tile[3] = plan[0] == 64 ? rotation(1, ceil_div64(N, plan[1]), plan[2], K) : 0;
   }
   return hipSuccess;
 }
