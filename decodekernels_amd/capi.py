@@ -235,9 +235,9 @@ def gemm_plan(M: int, N: int, K: int, with_workspace: bool = True) -> tuple[int,
 
 
 def gemm_tile(M: int, N: int, K: int, with_workspace: bool = True) -> tuple[int, int, int, int]:
-    """What runs gemm_tn's plan for this shape; host arithmetic only: (tile
-    rows, tile columns, K splits, K-walk rotation) of the tiled kernel, or the
-    skinny kernel's (waves along N, waves along K, K splits, 0)."""
+    """gemm_tn's launch plan with its K-walk rotation; host arithmetic only: the
+    first three numbers of ``gemm_plan`` and the slices of 64 columns by which
+    each column tile of the tiled kernel starts its walk later (0: none)."""
     out = (ctypes.c_int * 4)()
     rc = lib().dk_gemm_tn_tile(M, N, K, int(with_workspace), out)
     if rc != 0:

@@ -21,14 +21,12 @@
 //   in flight across the per-step barrier.
 // * LDS-DMA (M > 64, batched decode and prefill): A and B tiles go from HBM
 //   straight into LDS (buffer_load ... lds), bank-conflict-free XOR-swizzled,
-//   through a multi-stage ring; thirteen tile shapes from 256x256 down to 64x64.
-//   A plan per size sets the workspace and the most K splits; a time model
-//   picks the tile that runs it (kTileModel), so that batches of a few hundred
-//   rows still fill all 256 CUs. The output tile leaves through the freed
-//   ring, read back row by row for 16-byte stores. At M <= 64 its 64-row
-//   tiles (64 or 128 columns, K split) replace the skinny kernel from M = 32
-//   where they fill the CUs, for N > 32768 (decode_dma_plan), and where they
-//   measured faster at any M (decode_tile_plan).
+//   through a multi-stage ring; eleven tile shapes from 256x256 down to 64x64. A
+//   time model picks the tile and the K split of a call (kTileModel), so that
+//   batches of a few hundred rows still fill all 256 CUs. The output tile
+//   leaves through the freed ring, read back row by row for 16-byte stores. At
+//   M <= 64 its 64-row tiles (64 or 128 columns, K split) replace the skinny
+//   kernel where the model has them faster (decode_plan).
 #include <algorithm>
 #include <type_traits>
 
@@ -507,10 +505,10 @@ __device__ __forceinline__ void store_tile(const f32x4 (&acc)[TM][TN], u32x4* ld
     return;
   }
   constexpr int kChunks = 16 * TM * kNc;  // 16-byte chunks of a wave's tile
+  static_assert(kChunks % kWave == 0, "whole passes");
 #pragma unroll
-  for (int it = 0; it < (kChunks + kWave - 1) / kWave; ++it) {
+  for (int it = 0; it < kChunks / kWave; ++it) {
     const int idx = it * kWave + lane;
-    if (kChunks % kWave != 0 && idx >= kChunks) break;  // last pass part-filled (192 x 224: 10.5 passes)
     const int row = idx / kNc;
     const int c = idx % kNc;
     const u32x4 val = *reinterpret_cast<const u32x4*>(stg + row * kPitch + c * 16);
@@ -538,9 +536,8 @@ __device__ __forceinline__ void ring_tile(const uint16_t* __restrict__ A, const 
   constexpr int TM = BM / WM / 16;  // 16-row fragments per wave
   constexpr int TN = BN / WN / 16;
   constexpr int LA = BM / 8 / NW;   // 1 KB DMA loads per wave per slice
-  // B's 8-row load groups need not divide among the waves (256 x 224: 28 groups
-  // for 8 waves). A wave past the last group skips its final load where the
-  // ring's waits are vmcnt(0) (2 stages); else it issues one that moves nothing,
+  // B's 8-row load groups need not divide among the waves (128 x 160: 20 groups
+  // for 8 waves). A wave past the last group issues a load that moves nothing,
   // aimed at a spare 1 KB, so that every wave has the same count in flight.
   constexpr int kGroupsB = BN / 8;
   constexpr int LB = (kGroupsB + NW - 1) / NW;
@@ -549,8 +546,7 @@ __device__ __forceinline__ void ring_tile(const uint16_t* __restrict__ A, const 
   static_assert(BM % (8 * NW) == 0 && BN % 8 == 0 && TM >= 1 && TN >= 1 && BN % (16 * WN) == 0, "tile shape");
   static_assert(STAGES >= 2 && (STAGES - 2) * (LA + LB) < 64, "vmcnt range");
   constexpr int kStageWave = stage_bytes<TM, TN>();
-  constexpr bool kSpare = kTailB && STAGES > 2;
-  constexpr int kRingU4 = STAGES * kSlice + (kSpare ? 64 : 0);
+  constexpr int kRingU4 = STAGES * kSlice + (kTailB ? 64 : 0);
   constexpr int kLdsU4 = kRingU4 > NW * kStageWave / 16 ? kRingU4 : NW * kStageWave / 16;
   static_assert(kLdsU4 * 16 <= 160 * 1024, "LDS of one workgroup (gfx950: 160 KB)");
   __shared__ u32x4 lds[kLdsU4];
@@ -606,8 +602,7 @@ __device__ __forceinline__ void ring_tile(const uint16_t* __restrict__ A, const 
   // steps with the walk (a compare and a select per slice). With the K offset
   // as the loads' scalar offset instead, as in the ping-pong body, the larger
   // tiles were 1-6% slower (us): 128 x 128 at M, N, K = 192, 16384, 3072 36.4
-  // against 34.3 and at 768, 3584, 3584 36.5 against 34.9, 192 x 224 at 768,
-  // 28672, 4096 177 against 168.
+  // against 34.3 and at 768, 3584, 3584 36.5 against 34.9.
   auto issue = [&](bool checked, int k0, int buf) {
     u32x4* base = lds + buf * kSlice;
     const unsigned out = checked && k0 + kc >= ke ? kNowhere : 0;  // or-ed in: a choice per load became a branch
@@ -620,10 +615,7 @@ __device__ __forceinline__ void ring_tile(const uint16_t* __restrict__ A, const 
 #pragma unroll
     for (int j = 0; j < LB; ++j) {
       u32x4* to = base + BM * 8 + (wave + j * NW) * 64;
-      if (kTailB && j == LB - 1 && wave + j * NW >= kGroupsB) {  // past B's last load group (offb is out of range)
-        if (!kSpare) break;
-        to = lds + STAGES * kSlice;
-      }
+      if (kTailB && j == LB - 1 && wave + j * NW >= kGroupsB) to = lds + STAGES * kSlice;  // (offb is out of range)
       const int off = static_cast<int>((offb[j] + 2 * k0) | out);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (__attribute__((address_space(3))) void*)to, 16, off, 0,
                                                0, 0);
@@ -960,14 +952,8 @@ __device__ __forceinline__ void ping_pong_tile(const uint16_t* __restrict__ A, c
                                 part);
 }
 
-// 2-stage tiles whose halves split into 16-row and 16-column fragments for 8
-// waves run the ping-pong body (256 x 256, 256 x 192, 192 x 256, 256 x 128,
-// 128 x 256; not 256 x 224 and 192 x 224), the others the ring.
-template <int BN, int STAGES>
-constexpr bool ping_pong() {
-  return STAGES == 2 && BN % 64 == 0;
-}
-
+// 2-stage tiles (256 x 256, 256 x 192, 192 x 256, 256 x 128, 128 x 256) run the
+// ping-pong body, the others the ring.
 // Two waves per SIMD as the register target, also where the LDS allows one: with
 // the whole register file the compiler keeps the sums of the 4-wave tiles in
 // accumulation registers and moves them back and forth each slice (64 x 64: 36
@@ -981,7 +967,7 @@ __global__ __launch_bounds__(WM * WN * kWave, 2) void gemm_dma_kernel(const uint
                                                                    uint16_t* __restrict__ C, int M, int N, int K,
                                                                    int lda, int ldb, int ldc, int vec_store,
                                                                    float* __restrict__ part, int k_split, unsigned rot_inv) {
-  if constexpr (ping_pong<BN, STAGES>())
+  if constexpr (STAGES == 2)
     ping_pong_tile<E, BM, BN, WM, WN>(A, B, bias, C, M, N, K, lda, ldb, ldc, vec_store, part, k_split, rot_inv);
   else
     ring_tile<E, BM, BN, WM, WN, STAGES>(A, B, bias, C, M, N, K, lda, ldb, ldc, vec_store, part, k_split, rot_inv);
@@ -1014,16 +1000,15 @@ hipError_t launch_dma(const uint16_t* A, const uint16_t* B, const uint16_t* bias
 using DmaLauncher = hipError_t (*)(const uint16_t*, const uint16_t*, const uint16_t*, uint16_t*, int, int, int, int,
                                    int, int, hipStream_t, float*, int, int, bool, int);
 
-// Launchers of kTileShapes' tile shapes, in the same order. The waves of the
-// 256 x 256 tile form a 2 x 4 grid (0-2% faster than 4 x 2).
+// Launchers of kTiles' tile shapes, in the same order. The waves of the 256 x
+// 256 tile form a 2 x 4 grid (0-2% faster than 4 x 2).
 template <typename E>
 const DmaLauncher* tile_launchers() {
   static const DmaLauncher fns[] = {
       launch_dma<E, 256, 256, 2, 4, 2>, launch_dma<E, 256, 192, 4, 2, 2>, launch_dma<E, 192, 256, 2, 4, 2>,
       launch_dma<E, 256, 128, 4, 2, 2>, launch_dma<E, 128, 256, 2, 4, 2>, launch_dma<E, 128, 128, 4, 2, 3>,
       launch_dma<E, 128, 160, 4, 2, 4>, launch_dma<E, 128, 64, 2, 2, 4>,  launch_dma<E, 64, 64, 2, 2, 4>,
-      launch_dma<E, 64, 128, 2, 2, 4>,  launch_dma<E, 192, 192, 4, 2, 3>, launch_dma<E, 192, 224, 4, 2, 2>,
-      launch_dma<E, 256, 224, 4, 2, 2>,
+      launch_dma<E, 64, 128, 2, 2, 4>,  launch_dma<E, 192, 192, 4, 2, 3>,
   };
   return fns;
 }
@@ -1061,6 +1046,7 @@ inline SkinnyPlan skinny_plan_wide(int M, int N, int K) {
 
 // Workgroup shapes (WN, WK) of the plans below, narrowest first.
 constexpr int kSkinnyShapes[][2] = {{1, 8}, {2, 4}, {4, 2}, {6, 2}, {7, 2}, {8, 1}};
+constexpr int kSkinnyShapeCount = static_cast<int>(sizeof(kSkinnyShapes) / sizeof(kSkinnyShapes[0]));
 constexpr int kSkinnyCus = 256;
 
 // The widest unsplit grid that fits one workgroup per CU (the narrowest shape
@@ -1095,20 +1081,8 @@ inline SkinnyPlan skinny_plan_unsplit(int M, int N, int K) {
 //     bytes) of activations, or failing that the fewest activation bytes;
 //  3. else the unsplit grid of 1, or for N > 32768 (no grid of one workgroup
 //     per CU) the wide plan.
-// Picks (waves along N x along K, splits), with the unsplit K-walk rotation;
-// us cold, interleaved with hipBLASLt, ratio to it:
-//   qkv (N 6144, K 4096): M <= 32 2 x 4 unsplit, 14.4 (M=1, 0.86x) ... 18.7
-//     (M=32, 1.05x); M = 48/64 6 x 2 with 4 splits, 21.3 (M=64, 1.00x);
-//   o (N 4096): M <= 32 1 x 8 unsplit, 11.3 ... 14.6 (0.62 ... 0.93x);
-//     M = 48/64 4 x 2 with 4 splits, 16.6 (M=64, 0.93x);
-//   gate_up (N 28672): 7 x 2 unsplit, 43.9 (M=1, 0.71x) ... 51.4 (M=64, 0.92x);
-//   down (N 4096, K 14336): M <= 8 1 x 8, 24.4 (0.88x); M = 16 / 32 2 x 4 / 4 x 2
-//     with 2 / 4 splits, 29.3 (M=32, 0.86x); M = 48/64 8 x 1 with 8 splits,
-//     33.0 (M=64, 0.65x).
-// Each pick was the fastest candidate of its shape and M, except gate_up at
-// M <= 32 before the rotation: there 4 x 2 (448 workgroups) was 6-8% faster on
-// one of four machines and 7 x 2 7% faster on two. A 257th workgroup puts two
-// on one CU and doubles that CU's time.
+// A 257th workgroup puts two on one CU and doubles that CU's time. Where 64-row
+// tiles are faster, they run instead (decode_plan).
 inline SkinnyPlan skinny_plan(int M, int N, int K, bool split_ok) {
   constexpr int64_t kKiB = 1024;
   SkinnyPlan u = skinny_plan_unsplit(M, N, K);
@@ -1120,7 +1094,7 @@ inline SkinnyPlan skinny_plan(int M, int N, int K, bool split_ok) {
       int wn, wk, splits, k_split;
       int64_t wgs;
     };
-    Cand cand[sizeof(kSkinnyShapes) / sizeof(kSkinnyShapes[0]) * 7];
+    Cand cand[kSkinnyShapeCount * 7];
     int nc = 0;
     int64_t max_wgs = 0;
     for (const auto& sh : kSkinnyShapes) {
@@ -1167,144 +1141,18 @@ inline SkinnyPlan skinny_plan(int M, int N, int K, bool split_ok) {
   return u.wn > 0 ? u : skinny_plan_wide(M, N, K);
 }
 
-inline int64_t skinny_workspace_bytes(const SkinnyPlan& p, int M, int N) {
+// What a call runs: tile `shape` of kTiles, or (shape < 0) the skinny kernel
+// with wn x wk waves; K split over workgroup rows of k_split columns.
+struct Plan {
+  int shape, wn, wk, splits, k_split, rot_step;
+};
+
+// Largest split-K workspace a tiled plan asks for (bytes); larger splits are not considered.
+constexpr int64_t kMaxWorkspace = int64_t{64} << 20;
+
+inline int64_t plan_workspace_bytes(const Plan& p, int M, int N) {
   return p.splits > 1 ? static_cast<int64_t>(p.splits) * M * N * static_cast<int64_t>(sizeof(float)) : 0;
 }
-
-// Plan of the LDS-DMA kernel (M > 64): tile shape and, with a workspace, K
-// split over workgroup rows. Time model fitted to interleaved cold timings of
-// every shape x {1, 2, 4, 8} splits on the Llama-3-8B projections at M = 128,
-// 256 and 512 (mean 1.5% from the fastest, picks identical to the previous
-// unsplit model at M >= 1000):
-//   rounds(tiles x splits over 256 CUs) x tile flops per split / rate(shape)
-//   + [splits > 1] (1.84 us + splits x M x N x 8 B / 4.68 TB/s),
-// the last term the fp32 partials written and read back plus the reduce
-// launch. Splits are considered only when the unsplit grid leaves CUs idle
-// (< 256 tiles). Measured (us, cold): down (N 4096, K 14336) M = 128 73.2 ->
-// 36.6 (128 x 128, 8 splits; hipBLASLt 83.6), M = 256 73.3 -> 50.9 (256 x 128,
-// 8; 69.0), M = 512 105.3 -> 75.8 (256 x 128, 4; 100.4); o M = 128 24.6 ->
-// 19.3 (64 x 64, 2); qkv M = 256 35.8 -> 33.5 (128 x 128, 2). The 256 x 192
-// tile (rate placed between its neighbours from the qkv M = 4096 timing) fills
-// whole rounds where 256 x 256 leaves the last one part-empty: qkv (N 6144)
-// M = 1536 / 3072 / 4096 / 6000 103.9 / 188.3 / 194.1 / 298.7 -> 93.5 / 175.7
-// / 182.2 / 258.1, N 3072 and 5120 at M = 4096 105.2 / 185.9 -> 98.3 / 175.3
-// (each pick the fastest of the three 256-row tiles). The 256 x 224 tile does
-// the same for N = 28672 (128 column tiles; its rate fitted to gate_up at
-// M = 384 ... 4096, where 256 x 256 leaves the last round part-empty):
-// gate_up M = 384 / 512 / 1024 / 1536 / 2048 / 3072 102.7 / 110.0 / 206.7 /
-// 306.0 / 411.7 / 604.3 -> 96.9 / 104.3 / 197.0 / 289.5 / 378.0 / 570.7 (at
-// M = 768 it ties 256 x 192, and the 192 x 224 tile below beats both; M = 4096
-// keeps 256 x 256, measured faster).
-// The 192 x 192 tile (8 waves, 3 stages; N = 6144 is 32 of its columns, so
-// M = 1536 is one full round): its rate is the one, on a grid search over
-// every (tile, split) candidate timed for six projections at M = 128 ... 6144,
-// that adds no pick more than 2% slower than the plan before it. It takes qkv
-// (N 6144) at M = 384 / 768 / 1536 / 3072 from 43.8 / 62.3 / 90.8 / 159.5 to
-// 38.0 / 53.6 / 70.8 / 133.1 us (hipBLASLt 40.1 / 52.8 / 78.1 / 141.0).
-// The 192 x 224 tile (2 stages, 106 KB; its last epilogue pass is half
-// filled) got its rate the same way, on eight projections (Qwen2.5-7B's
-// gate_up and down added): every rate in 4.51 ... 4.60 picks it for 12 shapes,
-// none more than 0.4% slower, and from 4.61 on it displaces 192 x 192 at
-// 7-32% cost. Gains: Llama gate_up M = 768 182.1 -> 166.1 us; Qwen2.5-7B down
-// M = 384 ... 6144 4.5-7.5%, gate_up M = 512 5%, o M = 3072 6%, qkv M = 2048 7%.
-struct DmaPlan {
-  int shape, splits, k_split;
-};
-
-// Largest split-K workspace the plan asks for (bytes); larger splits are not considered.
-constexpr int64_t kDmaMaxWorkspace = int64_t{64} << 20;
-
-struct DmaShape {
-  int bm, bn;
-  double rate;  // TFLOP/s per CU
-};
-constexpr DmaShape kDmaShapes[] = {
-    {256, 256, 5.355}, {256, 224, 4.95}, {256, 192, 5.15}, {256, 128, 4.776}, {192, 224, 4.55},
-    {192, 192, 3.95},  {128, 128, 3.48}, {128, 64, 2.398}, {64, 64, 2.007},
-};
-
-inline DmaPlan dma_plan(int M, int N, int K, bool split_ok) {
-  DmaPlan best{0, 1, K};
-  double best_t = -1.0;
-  for (int i = 0; i < static_cast<int>(sizeof(kDmaShapes) / sizeof(kDmaShapes[0])); ++i) {
-    const DmaShape& sh = kDmaShapes[i];
-    const int64_t tiles = ceil_div64(M, sh.bm) * ceil_div64(N, sh.bn);
-    for (int s = 1; s <= 8; s *= 2) {
-      int ks = K, sp = 1;
-      if (s > 1) {
-        if (!split_ok || tiles >= kSkinnyCus || K / s < 512) break;
-        const int per = (K + s - 1) / s;
-        ks = (per + kDmaBK - 1) / kDmaBK * kDmaBK;
-        sp = (K + ks - 1) / ks;
-        if (sp < 2) continue;
-        if (static_cast<int64_t>(sp) * M * N * static_cast<int64_t>(sizeof(float)) > kDmaMaxWorkspace) break;
-      }
-      const double rounds = static_cast<double>(ceil_div64(tiles * sp, kSkinnyCus));
-      double t = rounds * sh.bm * sh.bn * 2.0 * ks / 1e6 / sh.rate;
-      if (sp > 1) t += 1.84 + static_cast<double>(sp) * M * N * 8 / 4.68e6;
-      if (best_t < 0 || t < best_t) {
-        best = DmaPlan{i, sp, ks};
-        best_t = t;
-      }
-    }
-  }
-  return best;
-}
-
-inline int64_t dma_workspace_bytes(const DmaPlan& d, int M, int N) {
-  return d.splits > 1 ? static_cast<int64_t>(d.splits) * M * N * static_cast<int64_t>(sizeof(float)) : 0;
-}
-
-// Tile that runs a plan: of the shapes, with at most the plan's K splits -- so
-// its workspace holds them, and an unsplit plan stays unsplit and gives the
-// same bits with and without a workspace -- the one with the smallest modelled
-// time. Microseconds, with n slices of 64 columns per split and W workgroups:
-//   start + n x slice x rounds + tile x ceil(W / 256)
-//     + [split] (split + per_split x splits + splits x M x N x 8 B / partials),
-// joined as (t^4 + m^4)^(1/4) with the time m of the operands and the output
-// at `memory` bytes a microsecond. A part-filled round of 256 workgroups takes
-// part_fill to 1 of a full one (its workgroups get more of the memory), times
-// last_round behind full ones. The 64 x 64 tile is paced by the latency of a
-// slice: each of its rounds counts whole (0.20 / 0.36 / 0.56 us a slice with 1 /
-// 2 / 3 workgroups to a CU, however many CUs have them).
-struct TileModel {
-  double start, split, per_split, partials, memory, part_fill, last_round;
-};
-struct TileShape {
-  int bm, bn;
-  double slice_us, tile_us;
-  bool whole_rounds;
-};
-struct TilePlan {
-  int shape, splits, k_split, rot_step;
-};
-
-// M > 64. Fitted to 250 (M, N, K) of the Llama-3-8B, Qwen2.5-7B and
-// Qwen2.5-0.5B projections and fifteen other (N, K), M = 65 ... 4096, every
-// shape with 1, 2, 3, 4, 6 and 8 splits, calls on three sets of operands in
-// turn: the pick is 0.6% slower than the fastest choice on average (worst 24%,
-// N 10387, K 624) and 1.35x faster than hipBLASLt (geometric means). Against
-// the plan's own tile in the ring body (us): qkv_proj of Qwen2.5-7B (N 4608,
-// K 3584) at M = 1003 47.5 -> 36.9, Llama-3-8B gate_up at M = 1003 201 -> 178,
-// down at M = 1003 / 2048 118 / 215 -> 101 / 175.
-constexpr TileModel kTileModel{2.61, 1.42, 0.234, 7.27e6, 4.99e6, 0.62, 1.148};
-constexpr TileShape kTileShapes[] = {
-    {256, 256, 1.233, 5.10, false}, {256, 192, 1.026, 6.34, false}, {192, 256, 0.993, 5.64, false},
-    {256, 128, 0.820, 3.59, false}, {128, 256, 0.821, 4.25, false}, {128, 128, 0.516, 1.51, false},
-    {128, 160, 0.622, 2.77, false}, {128, 64, 0.344, 1.54, false}, {64, 64, 0.184, 0.83, true},
-    {64, 128, 0.368, 2.00, false}, {192, 192, 0.900, 6.00, false}, {192, 224, 1.134, 6.20, false},
-    {256, 224, 1.415, 5.91, false},
-};
-constexpr int kTileCount = static_cast<int>(sizeof(kTileShapes) / sizeof(kTileShapes[0]));
-constexpr int kTile64x64 = 8, kTile64x128 = 9;  // their places in kTileShapes
-
-// M <= 64, plans of three splits or more. Fitted to 57 (M, N, K), M = 1 ... 64:
-// 1.0% slower than the fastest choice on average, 9% faster than the plan's
-// own kernel (worst 8% slower: N 3584, K 18944 at M = 64, 30.0 -> 32.5). Llama-3-8B at M = 64: qkv 15.0 (64 x
-// 128, 4 splits) -> 13.6 us (64 x 64, 2); Qwen2.5-7B qkv at M = 1 / 64 11.2 / 13.1
-// -> 9.2 / 11.3; N 3072, K 8192 at M = 64 15.3 -> 13.7.
-constexpr TileModel kDecodeModel{2.4, 1.672, 0.222, 8.24e6, 6.393e6, 0.636, 1.0};
-constexpr TileShape kDecodeShapes[] = {{64, 64, 0.207, 0.519, true}, {64, 128, 0.370, 1.027, false}};
 
 // K-walk rotation (see gemm_skinny_lds_kernel): column tile j starts its walk
 // j slices in. With one tile row every weight byte is read by one workgroup,
@@ -1319,182 +1167,139 @@ inline int rotation(int64_t tiles_m, int64_t tiles_n, int splits, int K) {
   return splits == 1 && tiles_m == 1 && tiles_n >= 128 && K >= 1536 && K % kDmaBK == 0 ? 1 : 0;
 }
 
-inline TilePlan fastest_tile(const TileModel& m, const TileShape* shapes, int count, int M, int N, int K,
-                             int max_splits) {
-  TilePlan best{0, 1, K, 0};
-  double best_t = -1.0;
-  const double mn = static_cast<double>(M) * N;
-  const double mem = 2.0 * (static_cast<double>(M) * K + static_cast<double>(N) * K + mn) / m.memory;
-  const double mem4 = mem * mem * mem * mem;
-  for (int i = 0; i < count; ++i) {
-    const TileShape& sh = shapes[i];
-    const int64_t tiles_m = ceil_div64(M, sh.bm);
-    const int64_t tiles_n = ceil_div64(N, sh.bn);
-    for (const int s : {1, 2, 3, 4, 6, 8}) {
-      int ks = K;
-      if (s > 1) {
-        if (s > max_splits || tiles_m * tiles_n > kSkinnyCus || K / s < 512) break;
-        ks = ((K + s - 1) / s + kDmaBK - 1) / kDmaBK * kDmaBK;
-        if ((K + ks - 1) / ks != s) continue;  // every split non-empty
-      }
-      const int64_t wgs = tiles_m * tiles_n * s;
-      const double n = static_cast<double>((ks + kDmaBK - 1) / kDmaBK);
-      const int64_t full = wgs / kSkinnyCus;
-      const int64_t rem = wgs % kSkinnyCus;
-      double rounds = static_cast<double>(full);
-      if (rem > 0) {
-        const double part =
-            sh.whole_rounds ? 1.0 : m.part_fill + (1.0 - m.part_fill) * static_cast<double>(rem) / kSkinnyCus;
-        rounds += (full > 0 && !sh.whole_rounds ? m.last_round : 1.0) * part;
-      }
-      double t = m.start + n * sh.slice_us * rounds + sh.tile_us * static_cast<double>(full + (rem > 0 ? 1 : 0));
-      if (s > 1) t += m.split + m.per_split * s + s * mn * 8.0 / m.partials;
-      t = t * t * t * t + mem4;
-      if (best_t < 0 || t < best_t) {
-        best = TilePlan{i, s, ks, rotation(tiles_m, tiles_n, s, K)};
-        best_t = t;
-      }
-    }
-  }
-  return best;
-}
-
-inline TilePlan tile_plan(int M, int N, int K, int plan_splits) {
-  return fastest_tile(kTileModel, kTileShapes, kTileCount, M, N, K, plan_splits);
-}
-
-// The LDS-DMA kernel at decode sizes (M <= 64), on one 64-row tile: column
-// tiles of bn = 64 (4 waves, two workgroups per CU) or 128 (4 waves, one per
-// CU), K split over workgroup rows. Where it applies it replaces the skinny
-// plan; bn = 0 keeps the skinny kernel. Fitted to interleaved cold timings
-// of both kernels at M = 1 ... 64 on the Llama-3-8B, Qwen2.5-7B and
-// Qwen2.5-0.5B projections (every candidate below, bf16, with the split
-// reduce):
-//  * candidates: bn in {128, 64} x 1, 2, 4, 8 splits of >= 768 columns, at
-//    most 256 workgroups; the pick streams the fewest weight bytes per
-//    workgroup (bn x k_split), bn = 128 on a tie;
-//  * it replaces the skinny plan when M >= 32 and the pick fills at least half
-//    of the CUs: the skinny kernel's per-step activation work grows with M
-//    while the tile's stays flat. Llama-3-8B at M = 64: qkv 20.9 -> 18.7 us
-//    (128 x 4 splits), o 17.1 -> 14.9 (64 x 4), down 32.7 -> 30.1 (128 x 8);
-//    qkv at M = 32 18.7 -> 17.2 (hipBLASLt 18.0). Below M = 32 the skinny
-//    plans are 5-10% faster on the 8B shapes, and with fewer than 128
-//    workgroups (the 0.5B model's small matrices) at every M. An unsplit
-//    pick replaces only a skinny grid that leaves over a quarter of the CUs
-//    idle (0.5B gate_up, 152 workgroups: 12.8 -> 10.4 us at M = 64), not a
-//    full one (8B gate_up: 64 x 128 unsplit 56.4 against 51.8 us);
-//  * for N > 32768, where no skinny grid fits one workgroup per CU, 64 x 64
-//    unsplit at every M: Qwen2.5-7B gate_up (N 37888) 57.7 -> 56.0 us at
-//    M = 1, 80.3 -> 65.6 at M = 64. At N <= 32768 the skinny kernel's full
-//    one-per-CU grid stays (Llama-3-8B gate_up: 43.9 against 47.6 us).
-struct DecodeDmaPlan {
-  int bn, splits, k_split;
+// Time model that picks what a call runs, in us. A grid of W workgroups, each
+// of n slices of 64 columns, takes
+//   ceil(W / 256) x (n x slice + tile)
+// with `ragged` for `slice` where K % 64 != 0 (rows then start off 128-byte lines, and
+// a slice's row segments lie in two), and a K split adds
+//   split + splits x M x N x 8 B / partials
+// (the fp32 partials written and read back; times `odd` where N % 4 != 0, whose
+// partial rows are stored and read in 4-byte pieces). Candidates: every tile
+// shape with 1, 2, 3, 4, 6 and 8 splits (at least 512 columns each, at most 256
+// tiles and 768 workgroups, partials within kMaxWorkspace). Constants are fitted
+// for the best picks, not the best times (so `slice` and `tile` are no
+// measurements), to calls with weights and activations cold in every cache,
+// the state that a layer's weights are in. Fitted to three sets of operands in
+// turn, which the last-level cache holds up to 85 MB each, a model misjudges
+// HBM-bound calls: down of Llama-3-8B (N 4096, K 14336) at M = 64 / 256 took 30.7 /
+// 51.2 us with such picks (64 x 64 in 4 splits, 128 x 128 in 4), 29.6 / 48.7 with
+// these.
+struct TimeModel {
+  double split, partials, odd;
+};
+struct TileShape {
+  int bm, bn;
+  double slice_us, ragged_us, tile_us;
 };
 
-inline DecodeDmaPlan decode_dma_plan(int M, int N, int K, bool split_ok) {
-  DecodeDmaPlan none{0, 1, K};
-  if (M > 64 || K <= 0) return none;
-  if (skinny_plan_unsplit(M, N, K).wn == 0) return DecodeDmaPlan{64, 1, K};
-  if (M < 32) return none;
-  DecodeDmaPlan best = none;
-  int64_t best_bytes = -1, best_wgs = 0;
-  for (const int bn : {128, 64}) {
-    const int64_t tiles = ceil_div64(N, bn);
-    for (int s = 1; s <= 8; s *= 2) {
-      int ks = K, sp = 1;
-      if (s > 1) {
-        if (!split_ok) break;
-        const int per = (K + s - 1) / s;
-        ks = (per + kDmaBK - 1) / kDmaBK * kDmaBK;
-        sp = (K + ks - 1) / ks;
-        if (ks < 768) break;
-        if (sp < 2) continue;
-      }
-      if (tiles * sp > kSkinnyCus) break;
-      const int64_t bytes = static_cast<int64_t>(bn) * ks;
-      if (best_bytes < 0 || bytes < best_bytes) {
-        best = DecodeDmaPlan{bn, sp, ks};
-        best_bytes = bytes;
-        best_wgs = tiles * sp;
-      }
+inline double split_us(const TimeModel& m, int splits, int M, int N) {
+  if (splits == 1) return 0.0;
+  return m.split + splits * (static_cast<double>(M) * N) * 8.0 / m.partials * (N % 4 != 0 ? m.odd : 1.0);
+}
+
+// Takes the fastest of `best` (at best_t, if >= 0) and the candidates of tile shape `i` with costs `sh`.
+inline void try_tile(const TimeModel& m, const TileShape& sh, int i, int M, int N, int K, bool split_ok, Plan& best,
+                     double& best_t) {
+  const int64_t tiles_m = ceil_div64(M, sh.bm);
+  const int64_t tiles = tiles_m * ceil_div64(N, sh.bn);
+  for (const int s : {1, 2, 3, 4, 6, 8}) {
+    int ks = K;
+    if (s > 1) {
+      if (!split_ok || tiles > kSkinnyCus || tiles * s > 3 * kSkinnyCus || K / s < 512 ||
+          static_cast<int64_t>(s) * M * N * static_cast<int64_t>(sizeof(float)) > kMaxWorkspace)
+        break;
+      ks = ((K + s - 1) / s + kDmaBK - 1) / kDmaBK * kDmaBK;
+      if ((K + ks - 1) / ks != s) continue;  // every split non-empty
+    }
+    const double n = static_cast<double>((ks + kDmaBK - 1) / kDmaBK);
+    const double slice = K % kDmaBK == 0 ? sh.slice_us : sh.ragged_us;
+    const double t = static_cast<double>(ceil_div64(tiles * s, kSkinnyCus)) * (n * slice + sh.tile_us) +
+                     split_us(m, s, M, N);
+    if (best_t < 0 || t < best_t) {
+      best = Plan{i, 0, 0, s, ks, rotation(tiles_m, ceil_div64(N, sh.bn), s, K)};
+      best_t = t;
     }
   }
-  if (2 * best_wgs < kSkinnyCus) return none;
-  if (best.splits == 1) {
-    // Unsplit, a tile streams about the bytes per workgroup of the skinny
-    // kernel's full grid, which its 14-wave workgroups stream faster.
-    const SkinnyPlan u = skinny_plan_unsplit(M, N, K);
-    if (4 * ceil_div64(N, 16 * u.wn) >= 3 * kSkinnyCus) return none;
-  }
+}
+
+// M > 64. Fitted to 2252 (M, N, K): the projections of Llama-3-8B, Qwen2.5-7B,
+// Qwen2.5-0.5B and Phi-3 at M = 65 ... 4096 and 1300 drawn ones, every candidate
+// timed. The pick is 0.8% slower than the fastest candidate on average (1% on
+// sizes left out of a fit, 17% at most for a projection). Against a plan of nine
+// tiles in the ring body alone, fitted to three projections, 0.927 of the time
+// (geometric mean), more than 5% slower at 22 sizes (10% at most); against a
+// model fitted to warm calls whose splits that plan capped, 0.956, more than 5%
+// slower at 32 (16%).
+constexpr TimeModel kTileModel{2.7, 6.28e6, 3.53};
+constexpr TileShape kTiles[] = {
+    {256, 256, 1.18, 1.52, 9.44},   {256, 192, 0.962, 1.26, 10.7},  {192, 256, 0.971, 1.26, 9.13},
+    {256, 128, 0.716, 1.21, 6.41},  {128, 256, 0.883, 1.24, 7.19},  {128, 128, 0.509, 0.847, 4.19},
+    {128, 160, 0.638, 0.909, 6.5},  {128, 64, 0.395, 0.706, 2.53},  {64, 64, 0.283, 0.442, 1.33},
+    {64, 128, 0.365, 0.678, 5.48},  {192, 192, 0.894, 1.23, 6.33},
+};
+constexpr int kTileCount = static_cast<int>(sizeof(kTiles) / sizeof(kTiles[0]));
+constexpr int kTile64x64 = 8, kTile64x128 = 9;  // their places in kTiles
+
+inline Plan tile_plan(int M, int N, int K, bool split_ok) {
+  Plan best{0, 0, 0, 1, K, 0};
+  double best_t = -1.0;
+  for (int i = 0; i < kTileCount; ++i) try_tile(kTileModel, kTiles[i], i, M, N, K, split_ok, best, best_t);
   return best;
 }
 
-inline int64_t decode_dma_workspace_bytes(const DecodeDmaPlan& d, int M, int N) {
-  return d.bn > 0 && d.splits > 1 ? static_cast<int64_t>(d.splits) * M * N * static_cast<int64_t>(sizeof(float)) : 0;
+// M <= 64: the skinny plan or a 64-row tile of 64 (4 waves, two workgroups per
+// CU) or 128 columns (4 waves, one per CU). The skinny plan is modelled as
+//   1.26 + max(1, W / 256) x (n x step + base) [+ the split],
+// n slices per wave, `step` by workgroup shape (kSkinnyShapes) times a factor by
+// row tiles, `base` by row tiles (M <= 16, <= 32, <= 64). Where no skinny grid
+// fits one workgroup per CU (N > 32768), a tile runs at every M: of N 128256, K
+// 4096 at M = 16 the grid of 8 x 1 waves took 180 us, 64 x 128 177. Fitted like
+// kTiles, to 755 (M, N, K), M = 1 ... 64: the pick is 0.8% slower than the fastest
+// of the three kinds on average. Against a plan that took the fewest weight bytes per
+// workgroup from M = 32 on: 0.986 of the time, more than 5% slower at 15 sizes,
+// none of them a projection (2.4% at most). Llama-3-8B gate_up (N 28672, K
+// 4096) at M = 1 / 64 41.7 / 51.0 -> 39.9 / 43.8, head at M = 1 / 16 / 64 192 / 200 /
+// 221 -> 169 / 177 / 183.
+constexpr TimeModel kDecodeModel{2.37, 9.55e6, 8.76};
+constexpr TileShape kDecodeTiles[] = {{64, 64, 0.377, 0.377, 2.05}, {64, 128, 0.680, 0.680, 2.55}};
+constexpr double kSkinnyStep[] = {0.631, 0.527, 0.622, 0.764, 1.35, 0.589};  // as kSkinnyShapes
+constexpr double kSkinnyRows[] = {1.0, 1.59, 1.62};
+constexpr double kSkinnyBase[] = {1.71, 1.80, 2.53};
+
+inline Plan decode_plan(int M, int N, int K, bool split_ok) {
+  const SkinnyPlan p = skinny_plan(M, N, K, split_ok);
+  Plan best{-1, p.wn, p.wk, p.splits, p.k_split, 0};
+  if (K <= 0) return best;
+  double best_t = -1.0;
+  if (skinny_plan_unsplit(M, N, K).wn > 0) {
+    const int rows = p.mt / 2;  // row tiles 1, 2, 4
+    double step = 0.0;
+    for (int i = 0; i < kSkinnyShapeCount; ++i)
+      if (kSkinnyShapes[i][0] == p.wn) step = kSkinnyStep[i] * kSkinnyRows[rows];
+    const double n = static_cast<double>((p.k_split + kLdsBK - 1) / kLdsBK) / p.wk;
+    const double rounds = static_cast<double>(ceil_div64(N, 16 * p.wn) * p.splits) / kSkinnyCus;
+    best_t = 1.26 + std::max(1.0, rounds) * (n * step + kSkinnyBase[rows]) + split_us(kDecodeModel, p.splits, M, N);
+  }
+  try_tile(kDecodeModel, kDecodeTiles[0], kTile64x64, M, N, K, split_ok, best, best_t);
+  try_tile(kDecodeModel, kDecodeTiles[1], kTile64x128, M, N, K, split_ok, best, best_t);
+  return best;
 }
 
-// Tile that runs a decode plan (M <= 64) in place of its kernel; shape < 0:
-// none. Plans of three splits or more go to the faster of the two 64-row tiles
-// (kDecodeModel). Unsplit, a wide weight matrix is read fastest by 64-row
-// tiles with the K walks rotated; the lines are where the tiles fill the chip
-// (us, the plan's own kernel -> the tile, calls on three sets of operands in
-// turn; K < 2048 was not measured):
-//  * 64 x 64 when it has 192 to 256 tiles (two to a CU), over any plan: N 12288
-//    / 14336 / 16384 (K 4096) at M = 1 20.1 / 21.8 / 27.3 -> 17.5 / 20.5 / 24.4,
-//    at M = 64 24.4 / 29.8 / 35.3 -> 20.4 / 24.0 / 26.0; N 12288, K 6144 at M = 1
-//    29.3 against 29.9;
-//  * 64 x 128 when its last round fills 3/4 of the 256 CUs, over an unsplit
-//    plan: gate_up (N 28672, K 4096) M = 1 / 16 / 64 41.6 / 41.4 / 48.7 -> 39.5 /
-//    40.1 / 42.5, N 24576 at M = 1 35.9 -> 33.5, N 128256 at M = 1 / 16 / 64 194 /
-//    199 / 220 -> 171 / 176 / 182, N 57344 (K 8192) 169 -> 157. Below: N 20480
-//    (160 tiles, K 5120) 37.6 against 39.1, N 37888 (296) 52.7 against 60.
-inline TilePlan decode_tile_plan(int M, int N, int K, int plan_splits) {
-  const int64_t t128 = ceil_div64(N, 128);
-  const int64_t t64 = ceil_div64(N, 64);
-  if (K >= 2048 && t64 >= 192 && t64 <= kSkinnyCus) return TilePlan{kTile64x64, 1, K, rotation(1, t64, 1, K)};
-  if (K >= 2048 && plan_splits == 1 && t64 > kSkinnyCus &&
-      4 * t128 >= 3 * kSkinnyCus * ceil_div64(t128, kSkinnyCus))
-    return TilePlan{kTile64x128, 1, K, rotation(1, t128, 1, K)};
-  if (plan_splits < 3) return TilePlan{-1, 1, K, 0};
-  TilePlan t = fastest_tile(kDecodeModel, kDecodeShapes, 2, M, N, K, plan_splits);
-  t.shape = t.shape == 0 ? kTile64x64 : kTile64x128;
-  // At small M the skinny kernel's 5-6% lead at short K (us: N 5731, K 5496, M = 1
-  // 16.0 against 17.1; N 8765, K 5608, M = 2 22.8 against 24.3) turns with K (N
-  // 10240, K 8192, M = 1 39.0 against 32.5).
-  if (t.shape == kTile64x128 && M < 32 && K < 8192) return TilePlan{-1, 1, K, 0};
-  // Below half of the CUs the skinny kernel's narrower tiles read faster (N 896,
-  // K 4864, M = 6: 6.8 us against 8.8 with 56 workgroups).
-  return ceil_div64(N, kTileShapes[t.shape].bn) * t.splits >= kSkinnyCus / 2 ? t : TilePlan{-1, 1, K, 0};
-}
-
-// What a call of one size runs with a full workspace: the plan, the tile that
-// runs it, and the plan's workspace. A function of the sizes alone, kept per
-// thread in a small direct-mapped table: a call asks for it twice (workspace,
-// launch), and its evaluation (0.3-1 us of host time) shows where the kernel
-// takes less than its launch.
+// What a call of one size runs with the workspace of `full` and with less: a plan
+// that does not split is the same in both, so its results do not depend on the
+// workspace. A function of the sizes alone, kept per thread in a small
+// direct-mapped table: a call asks for it twice (workspace, launch), and its
+// evaluation (0.3-1 us of host time) shows where the kernel takes less than
+// its launch.
 struct CallPlan {
   int M, N, K;  // M = 0: an empty entry
-  int64_t workspace_bytes;
-  DmaPlan dma;             // M > 64
-  DecodeDmaPlan decode;    // M <= 64, and
-  SkinnyPlan skinny;       // where decode.bn = 0
-  TilePlan tile;
+  Plan full, unsplit;
 };
 
 inline CallPlan make_call_plan(int M, int N, int K) {
-  CallPlan c{M, N, K, 0, {}, {}, {}, {}};
-  if (M > 64) {
-    c.dma = dma_plan(M, N, K, true);
-    c.workspace_bytes = dma_workspace_bytes(c.dma, M, N);
-    c.tile = tile_plan(M, N, K, c.dma.splits);
-  } else {
-    c.decode = decode_dma_plan(M, N, K, true);
-    c.skinny = skinny_plan(M, N, K, true);
-    c.workspace_bytes =
-        c.decode.bn > 0 ? decode_dma_workspace_bytes(c.decode, M, N) : skinny_workspace_bytes(c.skinny, M, N);
-    c.tile = decode_tile_plan(M, N, K, c.decode.bn > 0 ? c.decode.splits : c.skinny.splits);
-  }
-  return c;
+  const auto plan = M > 64 ? tile_plan : decode_plan;
+  const Plan full = plan(M, N, K, true);
+  return CallPlan{M, N, K, full, full.splits > 1 ? plan(M, N, K, false) : full};
 }
 
 inline const CallPlan& call_plan(int M, int N, int K) {
@@ -1517,65 +1322,47 @@ template <typename E>
 hipError_t launch(const uint16_t* A, const uint16_t* B, const uint16_t* bias, uint16_t* C, int M, int N, int K,
                   int lda, int ldb, int ldc, void* workspace, int64_t workspace_bytes, hipStream_t s,
                   int* deferred_splits, bool dma_ok) {
-  if (M <= 64) {
-    const CallPlan& full = call_plan(M, N, K);
-    DecodeDmaPlan d = dma_ok ? full.decode : DecodeDmaPlan{0, 1, 0};
-    SkinnyPlan p = full.skinny;
-    TilePlan t = full.tile;
-    // A workspace smaller than the plan's needs runs exactly the plan
-    // without one (both kernels' choices then exclude splits).
-    const int64_t need = d.bn > 0 ? decode_dma_workspace_bytes(d, M, N) : skinny_workspace_bytes(p, M, N);
-    if (need > 0 && (workspace == nullptr || need > workspace_bytes)) {
-      if (dma_ok) d = decode_dma_plan(M, N, K, false);
-      p = skinny_plan(M, N, K, false);
-      t = decode_tile_plan(M, N, K, 1);
+  const auto fits = [&](const Plan& q) {
+    return q.splits == 1 || (workspace != nullptr && plan_workspace_bytes(q, M, N) <= workspace_bytes);
+  };
+  const CallPlan& c = call_plan(M, N, K);
+  Plan p = fits(c.full) ? c.full : c.unsplit;
+  if (!dma_ok) {
+    SkinnyPlan k = skinny_plan(M, N, K, true);
+    p = Plan{-1, k.wn, k.wk, k.splits, k.k_split, 0};
+    if (!fits(p)) {
+      k = skinny_plan(M, N, K, false);
+      p = Plan{-1, k.wn, k.wk, k.splits, k.k_split, 0};
     }
-    if (!dma_ok) t.shape = -1;
-    if (t.shape >= 0) {
-      if (deferred_splits != nullptr) *deferred_splits = t.splits;
-      return tile_launchers<E>()[t.shape](A, B, bias, C, M, N, K, lda, ldb, ldc, s,
-                                          t.splits > 1 ? static_cast<float*>(workspace) : nullptr, t.splits, t.k_split,
-                                          deferred_splits == nullptr, t.rot_step);
-    }
-    if (d.bn > 0) {
-      if (deferred_splits != nullptr) *deferred_splits = d.splits;
-      return tile_launchers<E>()[d.bn == 64 ? kTile64x64 : kTile64x128](
-          A, B, bias, C, M, N, K, lda, ldb, ldc, s, d.splits > 1 ? static_cast<float*>(workspace) : nullptr, d.splits,
-          d.k_split, deferred_splits == nullptr, rotation(1, ceil_div64(N, d.bn), d.splits, K));
-    }
-    float* part = p.splits > 1 ? static_cast<float*>(workspace) : nullptr;
-    if (deferred_splits != nullptr) *deferred_splits = p.splits;
-    const dim3 g2(static_cast<unsigned>(ceil_div64(N, 16 * p.wn)), static_cast<unsigned>(p.splits));
-#define DK_SKINNY_LDS(MT_, WN_, WK_)                                                                 \
-  case MT_ * 100 + WN_ * 10 + WK_:                                                                   \
+  }
+  if (deferred_splits != nullptr) *deferred_splits = p.splits;
+  float* part = p.splits > 1 ? static_cast<float*>(workspace) : nullptr;
+  if (p.shape >= 0)
+    return tile_launchers<E>()[p.shape](A, B, bias, C, M, N, K, lda, ldb, ldc, s, part, p.splits, p.k_split,
+                                        deferred_splits == nullptr, p.rot_step);
+  const dim3 g2(static_cast<unsigned>(ceil_div64(N, 16 * p.wn)), static_cast<unsigned>(p.splits));
+#define DK_SKINNY_LDS(MT_, WN_, WK_)                                                                                   \
+  case MT_ * 100 + WN_ * 10 + WK_:                                                                                     \
     hipLaunchKernelGGL((gemm_skinny_lds_kernel<E, MT_, WN_, WK_, DK_SKINNY_DEPTH>), g2, dim3(WN_ * WK_ * kWave), 0, s, \
-                       A, B, bias, C, M, N, K, lda, ldb, ldc, part, p.k_split);                            \
+                       A, B, bias, C, M, N, K, lda, ldb, ldc, part, p.k_split);                                        \
     break;
-#define DK_SKINNY_MT(MT_)                                                                                 \
-  DK_SKINNY_LDS(MT_, 1, 8) DK_SKINNY_LDS(MT_, 2, 4) DK_SKINNY_LDS(MT_, 4, 2) DK_SKINNY_LDS(MT_, 6, 2)     \
+#define DK_SKINNY_MT(MT_)                                                                             \
+  DK_SKINNY_LDS(MT_, 1, 8) DK_SKINNY_LDS(MT_, 2, 4) DK_SKINNY_LDS(MT_, 4, 2) DK_SKINNY_LDS(MT_, 6, 2) \
   DK_SKINNY_LDS(MT_, 7, 2) DK_SKINNY_LDS(MT_, 8, 1)
-    switch (p.mt * 100 + p.wn * 10 + p.wk) {
-      DK_SKINNY_MT(1)
-      DK_SKINNY_MT(2)
-      DK_SKINNY_MT(4)
-      default: return hipErrorInvalidValue;  // not a shape the plans produce
-    }
+  switch ((M <= 16 ? 1 : (M <= 32 ? 2 : 4)) * 100 + p.wn * 10 + p.wk) {
+    DK_SKINNY_MT(1)
+    DK_SKINNY_MT(2)
+    DK_SKINNY_MT(4)
+    default: return hipErrorInvalidValue;  // not a shape the plans produce
+  }
 #undef DK_SKINNY_MT
 #undef DK_SKINNY_LDS
-    if (part != nullptr && deferred_splits == nullptr) {
-      const hipError_t e = hipGetLastError();
-      if (e != hipSuccess) return e;
-      launch_splitk_reduce<E>(part, p.splits, M, N, bias, C, ldc, s);
-    }
-    return hipGetLastError();
+  if (part != nullptr && deferred_splits == nullptr) {
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    launch_splitk_reduce<E>(part, p.splits, M, N, bias, C, ldc, s);
   }
-  const CallPlan& full = call_plan(M, N, K);
-  const bool fits = full.workspace_bytes == 0 || (workspace != nullptr && full.workspace_bytes <= workspace_bytes);
-  const TilePlan t = fits ? full.tile : tile_plan(M, N, K, 1);
-  if (deferred_splits != nullptr) *deferred_splits = t.splits;
-  return tile_launchers<E>()[t.shape](A, B, bias, C, M, N, K, lda, ldb, ldc, s,
-                                      t.splits > 1 ? static_cast<float*>(workspace) : nullptr, t.splits, t.k_split,
-                                      deferred_splits == nullptr, t.rot_step);
+  return hipGetLastError();
 }
 
 }  // namespace gemm
@@ -1636,55 +1423,45 @@ extern "C" int dk_gemm_tn(int dtype, const void* A, const void* B, const void* b
 
 extern "C" int64_t dk_gemm_tn_workspace_bytes(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  return dk::gemm::call_plan(M, N, K).workspace_bytes;
+  return dk::gemm::plan_workspace_bytes(dk::gemm::call_plan(M, N, K).full, M, N);
 }
 
-extern "C" int dk_gemm_tn_plan(int M, int N, int K, int with_workspace, int* plan) {
+namespace {
+
+// The plan of a call; nullptr for sizes that are refused.
+const dk::gemm::Plan* plan_of(const char* op, int M, int N, int K, int with_workspace, const int* out) {
   dk::clear_error();
-  if (plan == nullptr) return dk::fail("gemm_tn_plan: plan must not be NULL");
-  if (M <= 0 || N <= 0 || K < 0) return dk::fail("gemm_tn_plan: M and N must be positive, K non-negative");
-  if (M > 64) {
-    const dk::gemm::DmaPlan d = dk::gemm::dma_plan(M, N, K, with_workspace != 0);
-    plan[0] = dk::gemm::kDmaShapes[d.shape].bm;
-    plan[1] = dk::gemm::kDmaShapes[d.shape].bn;
-    plan[2] = d.splits;
-    plan[3] = d.k_split;
-    return hipSuccess;
+  if (out == nullptr) {
+    dk::fail("%s: the output must not be NULL", op);
+    return nullptr;
   }
-  const dk::gemm::DecodeDmaPlan d = dk::gemm::decode_dma_plan(M, N, K, with_workspace != 0);
-  if (d.bn > 0) {
-    plan[0] = 64;
-    plan[1] = d.bn;
-    plan[2] = d.splits;
-    plan[3] = d.k_split;
-    return hipSuccess;
+  if (M <= 0 || N <= 0 || K < 0) {
+    dk::fail("%s: M and N must be positive, K non-negative", op);
+    return nullptr;
   }
-  const dk::gemm::SkinnyPlan p = dk::gemm::skinny_plan(M, N, K, with_workspace != 0);
-  plan[0] = p.wn;
-  plan[1] = p.wk;
-  plan[2] = p.splits;
-  plan[3] = p.k_split;
+  const dk::gemm::CallPlan& c = dk::gemm::call_plan(M, N, K);
+  return with_workspace != 0 ? &c.full : &c.unsplit;
+}
+
+}  // namespace
+
+extern "C" int dk_gemm_tn_plan(int M, int N, int K, int with_workspace, int* plan) {
+  const dk::gemm::Plan* p = plan_of("gemm_tn_plan", M, N, K, with_workspace, plan);
+  if (p == nullptr) return hipErrorInvalidValue;
+  plan[0] = p->shape >= 0 ? dk::gemm::kTiles[p->shape].bm : p->wn;
+  plan[1] = p->shape >= 0 ? dk::gemm::kTiles[p->shape].bn : p->wk;
+  plan[2] = p->splits;
+  plan[3] = p->k_split;
   return hipSuccess;
 }
 
 extern "C" int dk_gemm_tn_tile(int M, int N, int K, int with_workspace, int* tile) {
-  using namespace dk;
-  using namespace dk::gemm;
-  int plan[4];
-  if (tile == nullptr) return fail("gemm_tn_tile: tile must not be NULL");
-  if (const int rc = dk_gemm_tn_plan(M, N, K, with_workspace, plan)) return rc;
-  const TilePlan t = M > 64 ? tile_plan(M, N, K, plan[2]) : decode_tile_plan(M, N, K, plan[2]);
-  if (t.shape >= 0) {
-    tile[0] = kTileShapes[t.shape].bm;
-    tile[1] = kTileShapes[t.shape].bn;
-    tile[2] = t.splits;
-    tile[3] = t.rot_step;
-  } else {
-    tile[0] = plan[0];
-    tile[1] = plan[1];
-    tile[2] = plan[2];
-    tile[3] = plan[0] == 64 ? rotation(1, ceil_div64(N, plan[1]), plan[2], K) : 0;
-  }
+  const dk::gemm::Plan* p = plan_of("gemm_tn_tile", M, N, K, with_workspace, tile);
+  if (p == nullptr) return hipErrorInvalidValue;
+  tile[0] = p->shape >= 0 ? dk::gemm::kTiles[p->shape].bm : p->wn;
+  tile[1] = p->shape >= 0 ? dk::gemm::kTiles[p->shape].bn : p->wk;
+  tile[2] = p->splits;
+  tile[3] = p->rot_step;
   return hipSuccess;
 }
 

@@ -146,19 +146,20 @@ int64_t dk_gemm_tn_workspace_bytes(int M, int N, int K);
  * Launch plan of dk_gemm_tn_ws (with_workspace != 0, workspace large enough)
  * or dk_gemm_tn. Skinny kernel (M <= 64): plan[0..3] = waves along N per
  * workgroup (16 columns each), waves along K, K splits, columns per split;
- * tiled kernel (M > 64, and M <= 64 where 64-row tiles fill the CUs better:
- * plan[0] = 64) = tile rows, tile columns, K splits, columns per split. For
- * tests and tuning; launches nothing. The plan sets the workspace and the most
- * K splits a call may use; dk_gemm_tn_tile says which tile runs it.
+ * tiled kernel (M > 64, and M <= 64 where 64-row tiles are faster: plan[0] =
+ * 64) = tile rows, tile columns, K splits, columns per split. A plan that does
+ * not split is the same with and without a workspace. (At M <= 64 row strides
+ * of 2^22 elements or more rule the tiles out: the skinny kernel then runs.) For
+ * tests and tuning; launches nothing.
  * No counterpart in DecodeKernels.
  */
 int dk_gemm_tn_plan(int M, int N, int K, int with_workspace, int* plan);
 
 /*
- * What runs a plan: tile[0..3] = tile rows, tile columns, K splits (at most the
- * plan's) and K-walk rotation (slices of 64 columns per column tile) of the
- * tiled kernel, or, where the skinny kernel runs, the plan's first three
- * numbers and 0. For tests and tuning; launches nothing.
+ * The plan with its K-walk rotation: tile[0..2] = dk_gemm_tn_plan's first three
+ * numbers, tile[3] = slices of 64 columns by which each column tile of the tiled
+ * kernel starts its walk later (0: none). For tests and tuning; launches
+ * nothing.
  * No counterpart in DecodeKernels.
  */
 int dk_gemm_tn_tile(int M, int N, int K, int with_workspace, int* tile);

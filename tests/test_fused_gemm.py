@@ -10,12 +10,11 @@
 
 The unfused ops are each checked against the oracle by their own tests, so
 bit equality pins the fused ones to the oracle too. The shapes cover the
-plans that split K (skinny M <= 64 with 2 splits, the LDS-DMA kernel's
-64-row tiles at M = 32 ... 64 with 4 and 8 splits, its split plans at M = 128 /
-384 and, for qkv, 256), where the consumer sums the partial
-tiles itself -- asserted from the plan -- and plans that do not, where the
-fused call runs the two ops; plus rows the norm cannot vectorise (N not a
-multiple of 8: the two ops run), strided rows, bias, and both dtypes.
+plans that split K -- the split counts that run are asserted: 2 (skinny kernel
+and tiles), 3, 4, 6 and 8, each a kernel of its own in the norm -- where the
+consumer sums the partial tiles itself, and plans that do not, where the fused
+call runs the two ops; plus rows the norm cannot vectorise (N not a multiple of
+8: the two ops run), strided rows, bias, and both dtypes.
 """
 
 import pytest
@@ -32,31 +31,35 @@ EPS = 1e-5
 
 
 def _splits(M, N, K):
-    """K splits of gemm_tn's plan for this shape with a workspace."""
-    return capi.gemm_plan(M, N, K)[2]
+    """K splits that gemm_tn runs for this shape with a workspace."""
+    return capi.gemm_tile(M, N, K)[2]
 
 
 @pytest.mark.parametrize(
-    "M,N,K,split",
+    "M,N,K,splits",
     [
-        (64, 4096, 4096, True),    # o projection at batch 64: 4 splits (64 x 64 tiles)
-        (48, 4096, 4096, True),
-        (64, 4096, 14336, True),   # down projection at batch 64: 8 splits (64 x 128 tiles)
-        (32, 4096, 14336, True),   # 8 splits
-        (16, 4096, 14336, True),   # 2 splits
-        (8, 4096, 4096, False),
-        (1, 4096, 14336, False),
-        (128, 4096, 14336, True),  # LDS-DMA kernel, 8 splits
-        (384, 4096, 4096, True),   # LDS-DMA kernel, 2 splits
-        (256, 4096, 4096, False),
-        (1000, 4096, 4096, False),
+        (64, 4096, 4096, 4),    # o projection at batch 64: 64 x 64 tiles
+        (48, 4096, 4096, 4),
+        (64, 4096, 14336, 8),   # down projection at batch 64: 64 x 128 tiles
+        (32, 4096, 14336, 8),
+        (16, 4096, 14336, 2),   # the skinny kernel
+        (8, 4096, 4096, 1),
+        (1, 4096, 14336, 1),
+        (128, 4096, 14336, 8),  # 128 x 128 tiles
+        (384, 4096, 4096, 2),
+        (300, 3584, 3584, 3),
+        (300, 896, 4864, 3),    # 64 x 64 tiles
+        (67, 320, 3256, 6),
+        (384, 3584, 18944, 8),  # 192 x 256 tiles
+        (256, 4096, 4096, 1),
+        (1000, 4096, 4096, 1),
         (64, 4100, 4096, None),    # the norm has no vector path: the two ops
         (64, 2056, 1032, None),
     ],
 )
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("with_bias", [False, True])
-def test_gemm_add_rms_norm_equals_two_ops(M, N, K, split, dtype, with_bias):
+def test_gemm_add_rms_norm_equals_two_ops(M, N, K, splits, dtype, with_bias):
     g = torch.Generator(device="cuda").manual_seed(M * 7 + N + K)
     kw = dict(device="cuda", dtype=dtype)
     a = torch.randn(M, K, generator=g, **kw)
@@ -65,8 +68,8 @@ def test_gemm_add_rms_norm_equals_two_ops(M, N, K, split, dtype, with_bias):
     weight = (1 + 0.1 * torch.randn(N, generator=g, device="cuda")).to(dtype)
     # Residual and output rows padded past N (strided rows).
     resid0 = torch.randn(M, N + 24, generator=g, **kw)[:, :N]
-    if split is not None:
-        assert (_splits(M, N, K) > 1) == split
+    if splits is not None:
+        assert _splits(M, N, K) == splits
     ref_out = torch.empty(M, N + 8, **kw)[:, :N]
     ref_res = resid0.clone()
     torch.ops.decode_kernels.gemm_tn(ref_out, a, w, bias)
@@ -123,7 +126,7 @@ def _rope_case(M, hq, hkv, d, dtype, layout, fp8, seed):
     return kv, positions, slot_mapping, table
 
 
-@pytest.mark.parametrize("M", [8, 48, 64, 256])
+@pytest.mark.parametrize("M", [8, 48, 64, 256, 384])
 @pytest.mark.parametrize("is_neox", [True, False])
 @pytest.mark.parametrize("fp8", [False, True])
 def test_gemm_rotary_embedding_and_cache_equals_two_ops(M, is_neox, fp8):
@@ -147,7 +150,7 @@ def test_gemm_rotary_embedding_and_cache_equals_two_ops(M, is_neox, fp8):
     dk.gemm_rotary_embedding_and_cache(x, w, qkv2, hq, hkv, positions, d, table, is_neox, kc2, vc2, slot_mapping,
                                        bias=bias, **scales)
     torch.cuda.synchronize()
-    assert (_splits(M, N, hidden) > 1) == (M in (48, 64, 256))
+    assert _splits(M, N, hidden) == {8: 1, 48: 4, 64: 4, 256: 2, 384: 4}[M]
     assert torch.equal(qkv1, qkv2), "qkv rows differ from gemm_tn + rotary_embedding_and_cache"
     view = (lambda t: t.view(torch.uint8)) if fp8 else (lambda t: t)
     assert torch.equal(view(kv.k_cache), view(kc2)) and torch.equal(view(kv.v_cache), view(vc2)), "caches differ"

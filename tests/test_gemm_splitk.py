@@ -3,14 +3,14 @@
 
 Decode shapes run one workgroup per CU, with wide column tiles and, where
 that leaves too few tiles, the K reduction split over workgroups writing fp32
-partial tiles that a second kernel sums in a fixed order; from M = 32 (and
-for N > 32768) the LDS-DMA kernel's 64-row tiles take over where they fill
-the CUs. Checks: every (row tiles, workgroup shape, split or not) skinny plan
-and every (tile columns, split or not) decode DMA plan against the fp32
-oracle with a bias and a ragged N, in fp16 and bf16; every partial entry written
-(workspace pre-filled with NaN); determinism (two calls equal bit for bit); a
-missing or undersized workspace runs exactly ``dk_gemm_tn``; the torch op
-equals the C-ABI call; graph replays equal the eager result.
+partial tiles that a second kernel sums in a fixed order; the tiled kernel's
+64-row tiles take over where they are faster. Checks: every (row tiles,
+workgroup shape, split or not) plan of the skinny kernel and every (tile
+columns, split or not) decode tile against the fp32 oracle with a bias and a
+ragged N, in fp16 and bf16; every partial entry written (workspace pre-filled
+with NaN); determinism (two calls equal bit for bit); a missing or undersized
+workspace runs exactly ``dk_gemm_tn``; the torch op equals the C-ABI call; graph
+replays equal the eager result.
 """
 
 import ctypes
@@ -21,7 +21,7 @@ import torch
 import decodekernels_amd as dk
 from decodekernels_amd import capi
 from parity import assert_max_abs, gemm_f32
-from test_gemm_plan import COVERAGE_SHAPES, DECODE_DMA_SHAPES
+from test_gemm_plan import COVERAGE_SHAPES, DECODE_TILE_SHAPES, replica_skinny_plan, runs_tile
 
 pytestmark = pytest.mark.gpu
 
@@ -38,7 +38,7 @@ SPLIT_SHAPES = [
     (64, 4096, 4096),  # attention output projection: 64 x 64 tiles, 4 splits
     (48, 6144, 4096),  # fused qkv projection: 64 x 128 tiles, 4 splits
     (17, 1000, 8200),  # ragged N and K, the last split shorter
-    (33, 4101, 4104),  # N not a multiple of 4 (scalar reduce)
+    (33, 4101, 4104),  # 64 x 64 tiles, 3 splits, N not a multiple of 4 (scalar reduce)
     (64, 8, 1024),  # one N tile
     (1, 1536, 3072),  # 5 splits
     (16, 1280, 14336),  # 6 splits
@@ -66,7 +66,7 @@ def _ws_call(a, b, bias, c, ws, nbytes):
     _call(capi.lib().dk_gemm_tn_ws, a, b, bias, c, None if ws is None else ws.data_ptr(), nbytes)
 
 
-@pytest.mark.parametrize("M,N,K", COVERAGE_SHAPES + DECODE_DMA_SHAPES)
+@pytest.mark.parametrize("M,N,K", COVERAGE_SHAPES + DECODE_TILE_SHAPES)
 def test_every_plan_against_the_oracle(M, N, K):
     dtype = torch.bfloat16 if (M + N) % 2 else torch.float16
     a, b, bias = _operands(M, N, K, dtype, M * 131 + N)
@@ -77,6 +77,32 @@ def test_every_plan_against_the_oracle(M, N, K):
         c = torch.empty(M, N, device="cuda", dtype=dtype)
         _call(capi.lib().dk_gemm_tn, a, b, bias, c)
         assert_max_abs(c, gemm_f32(a, b, bias), dtype, f"gemm {M}x{N}x{K} unsplit")
+
+
+@pytest.mark.parametrize("M,N,K", [s for s in COVERAGE_SHAPES if runs_tile(capi.gemm_plan(*s)) or s[0] in (17, 33)])
+def test_skinny_plans_behind_wide_row_strides(M, N, K):
+    """The skinny kernel where the plan is a tile and the activations' row
+    stride is too large for the tiles' 32-bit offsets (2^22 elements): with a
+    workspace for its own K splits, and unsplit without one."""
+    dtype = torch.bfloat16 if (M + N) % 2 else torch.float16
+    a, b, bias = _operands(M, N, K, dtype, M * 137 + N)
+    rows = max(M, 2)  # a lone row's stride is not used
+    wide = torch.zeros(rows * (1 << 22), device="cuda", dtype=dtype).view(rows, 1 << 22)
+    wide[:M, :K] = a
+    if M < rows:
+        a = torch.cat([a, torch.zeros(rows - M, K, device="cuda", dtype=dtype)])
+    want = gemm_f32(a, b, bias)
+    wn, wk, splits, _ = replica_skinny_plan(rows, N, K)
+    print(f"gemm {rows}x{N}x{K}, row stride 2^22: {wn}x{wk} waves, {splits} splits", flush=True)
+    nbytes = 4 * splits * rows * N if splits > 1 else 0
+    ws = torch.full((max(nbytes // 4, 4),), float("nan"), device="cuda")
+    c = torch.empty(rows, N, device="cuda", dtype=dtype)
+    _ws_call(wide[:, :K], b, bias, c, ws, nbytes)
+    assert_max_abs(c, want, dtype, f"gemm {rows}x{N}x{K} {wn}x{wk} waves, {splits} splits")
+    if splits > 1:
+        assert not ws.isnan().any(), "a partial sum was not written"
+        _call(capi.lib().dk_gemm_tn, wide[:, :K], b, bias, c)
+        assert_max_abs(c, want, dtype, f"gemm {rows}x{N}x{K} unsplit")
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -108,12 +134,14 @@ TILED_SPLIT_SHAPES = [
     (128, 4096, 14336),  # 128 x 128 tiles, 8 splits
     (256, 4096, 14336),  # 256 x 128, 8 splits
     (512, 4096, 14336),  # 256 x 128, 4 splits
-    (128, 4096, 4096),  # 64 x 64, 2 splits
+    (128, 4096, 4096),  # 128 x 64, 4 splits
     (256, 6144, 4096),  # 128 x 128, 2 splits
-    (300, 4101, 4104),  # ragged M and N, N not a multiple of 4 (scalar partial stores and reduce)
+    (300, 4101, 4104),  # 128 x 160, 3 splits, ragged M and N, N not a multiple of 4 (scalar partial stores and reduce)
     (100, 1000, 8200),  # ragged K: the last split shorter
-    (65, 4096, 14336),
-    (961, 6113, 5704),  # 256 x 192 tiles, 2 splits, ragged M and N (scalar partial stores and reduce)
+    (65, 4096, 14336),  # 128 x 128, 8 splits
+    (300, 3584, 3584),  # 128 x 128, 3 splits
+    (67, 320, 3256),  # 64 x 64, 6 splits
+    (388, 5486, 7816),  # 256 x 192 tiles, 4 splits, ragged M and N (scalar partial stores and reduce)
 ]
 
 

@@ -1,104 +1,30 @@
-"""The tile that runs a gemm_tn plan (``dk_gemm_tn_tile``): the library's choice
-against a restatement of its time model on the CPU, and on the GPU one set of
-shapes per tile -- edges, remainders, short and ragged K, K splits, rotated
-walks -- against an fp32 GEMM at the parity bar.
-
-The plan (``dk_gemm_tn_plan``) sets the workspace and the most K splits; the
-tile keeps to both, so an unsplit plan runs unsplit whatever the tile.
+"""The tiles of gemm_tn, one set of sizes per tile -- edges, remainders, short and
+ragged K, K splits, rotated walks (``dk_gemm_tn_tile``) -- against an fp32 GEMM at
+the parity bar on the GPU; on the CPU, that each size runs the tile it stands for.
 """
 
 import ctypes
-import random
 
 import pytest
 import torch
 
 from decodekernels_amd import capi
-
-# (rows, columns, us per 64-column slice, us per tile, part-filled rounds count whole)
-TILES = [
-    (256, 256, 1.233, 5.10, False), (256, 192, 1.026, 6.34, False), (192, 256, 0.993, 5.64, False),
-    (256, 128, 0.820, 3.59, False), (128, 256, 0.821, 4.25, False), (128, 128, 0.516, 1.51, False),
-    (128, 160, 0.622, 2.77, False), (128, 64, 0.344, 1.54, False), (64, 64, 0.184, 0.83, True),
-    (64, 128, 0.368, 2.00, False), (192, 192, 0.900, 6.00, False), (192, 224, 1.134, 6.20, False),
-    (256, 224, 1.415, 5.91, False),
-]
-# start, split, per_split, partials, memory, part_fill, last_round
-MODEL = (2.61, 1.42, 0.234, 7.27e6, 4.99e6, 0.62, 1.148)
-DECODE_TILES = [(64, 64, 0.207, 0.519, True), (64, 128, 0.370, 1.027, False)]
-DECODE_MODEL = (2.4, 1.672, 0.222, 8.24e6, 6.393e6, 0.636, 1.0)
+from test_gemm_plan import TILES, random_shapes, runs_tile
 
 
-def _rotation(tiles_m, tiles_n, splits, K):
-    return 1 if splits == 1 and tiles_m == 1 and tiles_n >= 128 and K >= 1536 and K % 64 == 0 else 0
-
-
-def _fastest(model, tiles, M, N, K, max_splits, rounds_up=True):
-    start, split, per_split, partials, memory, part_fill, last_round = model
-    best, best_t = None, -1.0
-    mn = float(M) * N
-    mem = 2.0 * (float(M) * K + float(N) * K + mn) / memory
-    mem4 = mem * mem * mem * mem
-    for bm, bn, slice_us, tile_us, whole in tiles:
-        tm, tn = -(-M // bm), -(-N // bn)
-        for s in (1, 2, 3, 4, 6, 8):
-            ks = K
-            if s > 1:
-                if s > max_splits or tm * tn > 256 or K // s < 512:
-                    break
-                ks = -(-(-(-K // s)) // 64) * 64
-                if -(-K // ks) != s:
-                    continue
-            full, rem = divmod(tm * tn * s, 256)
-            rounds = float(full)
-            if rem > 0:
-                part = 1.0 if whole and rounds_up else part_fill + (1.0 - part_fill) * float(rem) / 256
-                rounds += (last_round if full > 0 and not whole else 1.0) * part
-            t = start + float(-(-ks // 64)) * slice_us * rounds + tile_us * float(full + (rem > 0))
-            if s > 1:
-                t += split + per_split * s + s * mn * 8.0 / partials
-            t = t * t * t * t + mem4
-            if best_t < 0 or t < best_t:
-                best, best_t = (bm, bn, s, _rotation(tm, tn, s, K)), t
-    return best
-
-
-def replica(M, N, K, with_workspace=True, **mistake):
-    plan = capi.gemm_plan(M, N, K, with_workspace)
-    if M > 64:
-        return _fastest(MODEL, TILES, M, N, K, plan[2], **mistake)
-    t64, t128 = -(-N // 64), -(-N // 128)
-    if K >= 2048 and 192 <= t64 <= 256:
-        return (64, 64, 1, _rotation(1, t64, 1, K))
-    if K >= 2048 and plan[2] == 1 and t64 > 256 and 4 * t128 >= 768 * -(-t128 // 256):
-        return (64, 128, 1, _rotation(1, t128, 1, K))
-    if plan[2] >= 3:
-        tile = _fastest(DECODE_MODEL, DECODE_TILES, M, N, K, plan[2], **mistake)
-        wide_ok = tile[1] == 64 or M >= 32 or K >= 8192
-        if wide_ok and -(-N // tile[1]) * tile[2] >= 128:
-            return tile
-    return (plan[0], plan[1], plan[2], _rotation(1, -(-N // plan[1]), plan[2], K) if plan[0] == 64 else 0)
-
-
-def _random_shapes(n, seed):
-    rng = random.Random(seed)
-    for _ in range(n):
-        M = rng.choice([rng.randint(1, 64), rng.randint(65, 600), rng.randint(65, 5000)])
-        N = rng.choice([rng.randint(1, 2000), rng.randint(1, 30000), rng.randint(12000, 130000)])
-        yield M, N, 8 * rng.choice([rng.randint(1, 64), rng.randint(1, 3000)])
-
-
-def test_library_picks_like_the_replica():
-    for M, N, K in _random_shapes(20000, 11):
+def test_tile_is_the_plan_and_its_rotation():
+    for M, N, K in random_shapes(10000, 11):
         for ws in (True, False):
-            tile = capi.gemm_tile(M, N, K, ws)
-            assert tile == replica(M, N, K, ws), (M, N, K, ws)
-            # within the plan's workspace, and unsplit where the plan is
-            assert tile[2] <= capi.gemm_plan(M, N, K, ws)[2]
+            tile, plan = capi.gemm_tile(M, N, K, ws), capi.gemm_plan(M, N, K, ws)
+            assert tile[:3] == plan[:3]
+            one_row = runs_tile(plan) and M <= plan[0] and -(-N // plan[1]) >= 128
+            assert tile[3] == (1 if one_row and plan[2] == 1 and K >= 1536 and K % 64 == 0 else 0), (M, N, K, ws)
 
 
-def test_planted_mistake_is_caught():
-    assert any(capi.gemm_tile(*s) != replica(*s, rounds_up=False) for s in _random_shapes(5000, 12))
+def test_every_tile_runs():
+    """Every compiled tile shape is picked, split and unsplit (the two of M <= 64 among them)."""
+    kinds = {(tile[:2], tile[2]) for tile in SHAPES}
+    assert kinds == {((bm, bn), split) for bm, bn, *_ in TILES for split in (False, True)}
 
 
 def test_tile_validation():
@@ -110,56 +36,63 @@ def test_tile_validation():
 # Tile, K splits, rotated -> shapes (M, N, K) that pick it: whole tiles, ragged M
 # and N (odd N: scalar stores), K of one to five slices, K ending inside a slice.
 SHAPES = {
-    (64, 64, False, 0): [(165, 1, 8), (84, 1, 152), (65, 131, 24), (1, 37488, 136), (1, 34369, 80), (1, 37679, 8)],
-    (64, 64, False, 1): [(24, 15886, 4672), (64, 15991, 2176), (59, 16292, 2688), (41, 38630, 2816)],
-    (64, 64, True, 0): [(103, 1, 1456), (65, 7, 1488), (103, 7, 2048), (1, 2720, 2712), (256, 320, 1504)],
-    (64, 128, False, 0): [
-        (32, 17749, 8), (34, 17000, 72), (33, 16549, 136), (33, 16524, 216), (33, 16706, 264), (135, 8301, 672),
-    ],
+    (64, 64, False, 0): [(165, 1, 8), (84, 1, 152), (17, 858, 88), (7, 15371, 280), (155, 1970, 248), (65, 131, 24)],
+    (64, 64, False, 1): [(32, 11709, 3328), (24, 15886, 4672), (64, 15991, 2176), (59, 16292, 2688), (41, 38630, 2816)],
+    (64, 64, True, 0): [(103, 1, 1456), (65, 7, 1488), (103, 7, 2048), (256, 320, 1504)],
+    (64, 128, False, 0): [(1, 37679, 8), (1, 34369, 80), (1, 37488, 136), (33, 16706, 264), (47, 17033, 256)],
     (64, 128, False, 1): [(1, 25857, 2624), (5, 25198, 4288), (23, 27676, 3712), (51, 27272, 3264)],
-    (64, 128, True, 0): [(1, 10240, 8192), (3, 10113, 8200), (32, 11709, 3328), (277, 1812, 5184)],
+    (64, 128, True, 0): [(24, 20752, 3456), (37, 19352, 2416), (18, 18702, 5264), (277, 1812, 5184), (55, 9179, 6392)],
     (128, 64, False, 0): [
-        (66, 9455, 8), (133, 5511, 8), (72, 8557, 72), (194, 4281, 136), (67, 8375, 136), (385, 2325, 16),
+        (66, 9455, 8), (385, 2325, 16), (72, 8557, 72), (67, 8375, 136), (71, 14183, 248), (340, 3703, 264),
     ],
-    (128, 64, False, 1): [(99, 9697, 1792), (111, 15145, 1728), (108, 10818, 3008), (123, 15164, 3584)],
-    (128, 64, True, 0): [(65, 4180, 3584), (68, 4201, 3528), (257, 1748, 4544), (640, 960, 5552)],
+    (128, 64, False, 1): [(99, 9697, 1792), (111, 15145, 1728), (123, 15164, 3584)],
+    (128, 64, True, 0): [(65, 4180, 3584), (68, 4201, 3528), (117, 5032, 3008), (210, 2638, 4192), (404, 1305, 4800)],
     (128, 128, False, 0): [
-        (72, 17476, 8), (157, 8460, 8), (257, 5486, 8), (67, 16867, 208), (137, 10887, 136), (132, 8229, 16),
+        (72, 17476, 8), (137, 10887, 136), (67, 16867, 208), (294, 10769, 112), (185, 11933, 304), (400, 5778, 5952),
     ],
     (128, 128, False, 1): [(101, 17903, 2432), (128, 28416, 1536), (120, 24116, 2112), (93, 26141, 3200)],
-    (128, 128, True, 0): [(67, 2898, 6488), (68, 2749, 6768), (86, 2747, 7168), (385, 2331, 3112), (256, 4352, 3360)],
+    (128, 128, True, 0): [(67, 2898, 6488), (68, 2749, 6768), (385, 2331, 3112), (131, 5511, 5312), (130, 6415, 6784)],
     (128, 160, False, 0): [
-        (66, 34011, 8), (140, 16583, 8), (67, 33182, 208), (1280, 3680, 6760), (72, 33510, 72), (129, 17819, 200),
+        (66, 34011, 8), (129, 17819, 200), (247, 19966, 96), (1851, 2337, 192), (244, 19598, 304), (135, 16573, 6528),
     ],
     (128, 160, False, 1): [(87, 32892, 2112), (118, 34385, 1792), (74, 39464, 2560), (98, 33702, 3712)],
-    (128, 160, True, 0): [(129, 5740, 4544), (131, 5511, 5312), (138, 6207, 4552), (1354, 1540, 5440)],
-    (128, 256, False, 0): [(263, 16610, 272), (264, 17761, 264), (257, 20614, 320), (259, 16199, 576)],
-    (128, 256, True, 0): [(66, 17103, 4984), (67, 16458, 5760), (69, 21476, 5912), (257, 5729, 6520)],
-    (192, 192, False, 0): [(130, 32809, 1288), (145, 33625, 1408), (1445, 12225, 392), (1397, 12206, 1152)],
-    (192, 192, False, 1): [(156, 35872, 2112), (136, 33759, 2752), (137, 39374, 2688), (160, 36479, 2816)],
-    (192, 192, True, 0): [(132, 8995, 5664), (136, 9479, 6848), (135, 16573, 6528), (1537, 2629, 6952)],
+    (128, 160, True, 0): [(138, 6207, 4552), (278, 3781, 4384), (66, 17103, 4984), (67, 16458, 5760)],
+    (128, 256, False, 0): [
+        (625, 12737, 16), (603, 12388, 112), (594, 13046, 136), (595, 12382, 1024), (638, 12664, 976),
+        (578, 12876, 2944),
+    ],
+    (128, 256, True, 0): [(66, 19156, 3248), (67, 21368, 5120), (69, 21476, 5912)],
+    (192, 192, False, 0): [
+        (132, 34762, 8), (129, 33092, 72), (293, 18540, 192), (263, 16610, 272), (279, 23607, 248), (131, 36961, 576),
+    ],
+    (192, 192, False, 1): [
+        (144, 39011, 1792), (156, 38208, 1728), (156, 35872, 2112), (136, 33759, 2752), (137, 39374, 2688),
+        (160, 36479, 2816),
+    ],
+    (192, 192, True, 0): [(129, 5740, 4544), (132, 8995, 5664), (257, 5729, 6520), (192, 11520, 6008)],
     (192, 256, False, 0): [
-        (129, 35791, 136), (275, 22700, 136), (131, 36961, 576), (384, 26880, 4104), (130, 34397, 208),
-        (259, 22417, 264),
+        (292, 32535, 8), (274, 27602, 96), (389, 16817, 264), (384, 29893, 152), (783, 10211, 240), (290, 28796, 304),
     ],
-    (192, 256, False, 1): [(144, 39011, 1792), (156, 38208, 1728), (186, 36458, 1536), (151, 39337, 1856)],
-    (192, 256, True, 0): [
-        (140, 5626, 6384), (137, 6259, 6432), (130, 6415, 6784), (192, 11520, 6008), (385, 8689, 6120),
-    ],
+    (192, 256, True, 0): [(133, 18632, 5312), (1295, 3784, 2824)],
     (256, 128, False, 0): [
-        (140, 32026, 72), (133, 22341, 136), (142, 25547, 576), (132, 23152, 264), (512, 16256, 128),
-        (257, 14131, 248),
+        (208, 29413, 40), (203, 24821, 104), (132, 23152, 264), (213, 29248, 136), (171, 30010, 248),
+        (197, 26551, 248),
     ],
-    (256, 128, False, 1): [(205, 22543, 2048), (179, 26269, 2560), (231, 22504, 3200), (226, 32416, 2688)],
-    (256, 128, True, 0): [(134, 7203, 6136), (135, 7240, 6720), (728, 2925, 5184), (230, 13347, 7024)],
+    (256, 128, False, 1): [
+        (204, 23697, 4480), (205, 22543, 2048), (213, 20560, 4416), (226, 32416, 2688), (231, 22504, 3200),
+        (215, 20556, 4544),
+    ],
+    (256, 128, True, 0): [(1615, 880, 5632), (1354, 1540, 5440), (251, 10593, 6920)],
     (256, 192, False, 0): [
-        (196, 33045, 784), (195, 34882, 832), (390, 22181, 840), (256, 35904, 896), (407, 22700, 896),
+        (238, 32773, 288), (256, 35904, 896), (199, 33686, 576), (229, 38988, 280), (196, 33045, 784),
+        (195, 34882, 832),
     ],
     (256, 192, False, 1): [(200, 36411, 1792), (208, 37390, 1984), (256, 39090, 1728), (244, 35619, 2176)],
-    (256, 192, True, 0): [(385, 5706, 5344), (386, 5459, 5640), (400, 5778, 5952), (204, 23697, 4480)],
-    (256, 256, False, 0): [
-        (392, 25337, 8), (129, 33092, 72), (265, 21840, 80), (389, 16817, 264), (257, 22915, 88), (199, 33686, 576),
+    (256, 192, True, 0): [
+        (386, 5612, 5696), (210, 11528, 6016), (197, 12064, 6376), (201, 11225, 7096), (1730, 1600, 6704),
     ],
+    (256, 256, False, 0): [(392, 25337, 8), (434, 29246, 104), (227, 35369, 208), (1162, 9994, 144), (400, 27892, 296)],
+    (256, 256, True, 0): [(194, 16468, 4128), (221, 16860, 4376), (197, 20604, 4904), (1280, 3680, 6760)],
 }
 
 
@@ -201,8 +134,8 @@ def test_tile_against_fp32(tile, bf16):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("tile, shape", [((64, 64), (192, 3008, 16)), ((128, 160), (1280, 3680, 6760)),
-                                         ((256, 128), (512, 16256, 128)), ((256, 256), (257, 22915, 88))])
+@pytest.mark.parametrize("tile, shape", [((64, 64), (192, 3008, 16)), ((128, 160), (129, 17816, 200)),
+                                         ((256, 128), (132, 23152, 264)), ((256, 256), (392, 25336, 8))])
 def test_output_rows_of_any_alignment(tile, shape):
     """Stores of 16, 8, 4 and 2 bytes: output rows of every stride modulo 8
     starting at every element offset modulo 8, odd and even N; the elements
