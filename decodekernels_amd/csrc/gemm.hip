@@ -602,23 +602,27 @@ __device__ __forceinline__ void ring_tile(const uint16_t* __restrict__ A, const 
   // steps with the walk (a compare and a select per slice). With the K offset
   // as the loads' scalar offset instead, as in the ping-pong body, the larger
   // tiles were 1-6% slower (us): 128 x 128 at M, N, K = 192, 16384, 3072 36.4
-  // against 34.3 and at 768, 3584, 3584 36.5 against 34.9.
+  // against 34.3 and at 768, 3584, 3584 36.5 against 34.9. The uneven 128 x 160
+  // tile keeps the scalar offset: at 1003, 4608, 3584 38.2 against 41.0 with warm
+  // weights, though 43.4 against 42.5 with cold ones.
+  constexpr bool kScalarK = kTailB;
   auto issue = [&](bool checked, int k0, int buf) {
+    const bool scalar = kScalarK && !checked;
     u32x4* base = lds + buf * kSlice;
     const unsigned out = checked && k0 + kc >= ke ? kNowhere : 0;  // or-ed in: a choice per load became a branch
 #pragma unroll
     for (int j = 0; j < LA; ++j) {
-      const int off = static_cast<int>((offa[j] + 2 * k0) | out);
+      const int off = static_cast<int>(scalar ? offa[j] : (offa[j] + 2 * k0) | out);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          ra, (__attribute__((address_space(3))) void*)(base + (wave + j * NW) * 64), 16, off, 0, 0, 0);
+          ra, (__attribute__((address_space(3))) void*)(base + (wave + j * NW) * 64), 16, off, scalar ? 2 * k0 : 0, 0, 0);
     }
 #pragma unroll
     for (int j = 0; j < LB; ++j) {
       u32x4* to = base + BM * 8 + (wave + j * NW) * 64;
       if (kTailB && j == LB - 1 && wave + j * NW >= kGroupsB) to = lds + STAGES * kSlice;  // (offb is out of range)
-      const int off = static_cast<int>((offb[j] + 2 * k0) | out);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (__attribute__((address_space(3))) void*)to, 16, off, 0,
-                                               0, 0);
+      const int off = static_cast<int>(scalar ? offb[j] : (offb[j] + 2 * k0) | out);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (__attribute__((address_space(3))) void*)to, 16, off,
+                                               scalar ? 2 * k0 : 0, 0, 0);
     }
   };
 
@@ -836,10 +840,10 @@ __device__ __forceinline__ void ping_pong_tile(const uint16_t* __restrict__ A, c
   // also for slices that end past the K range (or start there: nothing is moved).
   auto issue_a = [&](bool checked, int k0, int buf, int i) {
     u32x4* base = lds + buf * kSlice + i * kHalfA;
-    const unsigned out = k0 + kc < ke ? 0 : kNowhere;
+    const bool in = k0 + kc < ke;
 #pragma unroll
     for (int j = 0; j < LA; ++j) {
-      const int off = static_cast<int>(checked ? (offa[i][j] + 2 * k0) | out : offa[i][j]);
+      const int off = static_cast<int>(checked ? (in ? offa[i][j] + 2 * k0 : kNowhere) : offa[i][j]);
       u32x4* to = wave + j * NW < kGroupsA ? base + (wave + j * NW) * 64 : lds + 2 * kSlice;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (__attribute__((address_space(3))) void*)to, 16, off,
                                                checked ? 0 : 2 * k0, 0, 0);
@@ -847,10 +851,10 @@ __device__ __forceinline__ void ping_pong_tile(const uint16_t* __restrict__ A, c
   };
   auto issue_b = [&](bool checked, int k0, int buf, int i) {
     u32x4* base = lds + buf * kSlice + 2 * kHalfA + i * kHalfB;
-    const unsigned out = k0 + kc < ke ? 0 : kNowhere;
+    const bool in = k0 + kc < ke;
 #pragma unroll
     for (int j = 0; j < LB; ++j) {
-      const int off = static_cast<int>(checked ? (offb[i][j] + 2 * k0) | out : offb[i][j]);
+      const int off = static_cast<int>(checked ? (in ? offb[i][j] + 2 * k0 : kNowhere) : offb[i][j]);
       u32x4* to = wave + j * NW < kGroupsB ? base + (wave + j * NW) * 64 : lds + 2 * kSlice;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (__attribute__((address_space(3))) void*)to, 16, off,
                                                checked ? 0 : 2 * k0, 0, 0);
