@@ -1400,7 +1400,10 @@ void launch_reduce_sized(const KParams& kp, int num_seqs, hipStream_t stream) {
   // 54.1 -> 50.3; 4096 heads 187 -> 173; 1792 heads of 64 39.3 -> 33.9; 2048 heads
   // of 128, 64 x 16384 691 -> 684, one long 60.1 -> 53.1. At 512 heads one long
   // 49.8 -> 49.3 (256) and 24.8 -> 24.6 (128); below, 16 waves win there: 256
-  // heads of 256 48.2 against 48.7, 224 heads of 64 13.8 against 14.1.
+  // heads of 256 48.2 against 48.7, 224 heads of 64 13.8 against 14.1. The
+  // partition grid, whose heads really have a row per 512 tokens, gets here only
+  // at head_dim 64 with 32 streams of 16 heads and 64 rows: 16 and 4 waves within
+  // 2% (32 x 32768 tokens 56.0 / 55.2, one long 14.7 / 14.9).
   else if (entries < 64 || (PIECES && static_cast<int64_t>(kp.num_q_heads) * num_seqs >= 512))
     launch_reduce<D, 4, PIECES, E>(kp, num_seqs, stream);
   else launch_reduce<D, 16, PIECES, E>(kp, num_seqs, stream);
